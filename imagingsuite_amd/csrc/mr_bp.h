@@ -26,6 +26,7 @@ struct BpArgs {
     // 3 NearestNeighborBP; centeroffset and centerinc of the block
     int tilt;
     float tilt_co, tilt_ci;
+    const int *gate;     // LDS kernel without tilt: run only if *gate != 0 (NULL: always)
 };
 
 // Uploads the tables of n_proj projections (angles, weights) into the plan
@@ -48,5 +49,33 @@ int launch_bp_prep(const float *proj, float *sino, const int *idx, const float *
 // with slices % 4 != 0, whose second column is read at a different offset);
 // 1: LDS-staged tiles.  exact: the reference's float operation order.
 int run_bp(const BpArgs &a, int interp, int impl, int exact, hipStream_t s);
+
+// Matrix-core form of the fused mode (mr_bp_mfma.hip).
+struct BpmArgs {
+    const unsigned *split;   // split samples [k][pair][zt][plane][16] (launch_bp_split_prep)
+    float *vol;
+    const float4 *tab;       // as BpArgs
+    const int2 *mask;
+    const float2 *scale;     // per slice: factor on the samples, its inverse
+    const int *flag;         // set: the samples do not fit the split, the kernel leaves at once
+    int nu, nv, vp, npair, nk, nz4;   // vp: slices rounded up to 16; npair: column pairs
+    int chain;               // 1: the volume holds the sums of earlier projections, continue them
+    int ntx, nty, ntz, zt0, sw;
+};
+// Voxel tile of the matrix-core kernel for a stack with nk used projections,
+// or false where the VALU kernel serves it.
+bool bpm_shape(int nu, int nv, int nk, int &tile);
+inline int bpm_vp(int nv) { return (nv + 15) & ~15; }
+inline int bpm_npair(int nu) { return (nu + 1) / 2; }
+size_t bpm_part_words(size_t nv, size_t nk);   // words of launch_bp_scale's partial maxima
+int launch_bp_scale(const float *proj, const int *idx, const float *wts, int nu, int nv, int nk, unsigned *part,
+                    float2 *scale, int *flag, hipStream_t s);
+int launch_bp_split_prep(const BpmArgs &a, const float *proj, const int *idx, const float *wts, int vpad,
+                         hipStream_t s);
+int run_bpm(const BpmArgs &a, int tile, hipStream_t s);
+// Persistent launch over a batch's items (bp_mfma_batch_kernel).
+int bpm_batch_grid(int &grid);
+int launch_bpm_batch(const BpmArgs *d_stacks, const int4 *d_items, const int *d_parts, int *d_counters, int grid,
+                     hipStream_t s);
 
 }  // namespace mr

@@ -605,6 +605,7 @@ __global__ __launch_bounds__(256) void bp_lds_kernel(BpArgs a)
 {
     __shared__ float sm[KC][kBpSpan][ZT + 4];
     __shared__ int sb0[KC];
+    if (a.gate && *a.gate == 0) return;
     int bx, by, bz;
     if (!tile_of_block(a, bx, by, bz)) return;
     bp_lds_tile<ZT, INTERP, EXACT, KC, PIPE>(a, bx, by, bz, sm, sb0);
@@ -632,8 +633,15 @@ __global__ __launch_bounds__(256) void bp_lds_tilt_kernel(BpArgs a)
 template <int ZT, int INTERP, bool EXACT, int KC>
 __global__ __launch_bounds__(256) void bp_batch_kernel(const BpArgs *__restrict__ stacks,
                                                        const int4 *__restrict__ items,
-                                                       const int *__restrict__ part_begin, int *counters)
+                                                       const int *__restrict__ part_begin, int *counters,
+                                                       const int *__restrict__ flags, int n_stacks)
 {
+    if (flags) {
+        // only the stacks whose samples did not fit the matrix-core form
+        int any = 0;
+        for (int i = threadIdx.x; i < n_stacks; i += 256) any |= flags[i];
+        if (!__syncthreads_or(any)) return;
+    }
     __shared__ float sm[KC][kBpSpan][ZT + 4];
     __shared__ int sb0[KC];
     __shared__ int item;
@@ -653,10 +661,12 @@ __global__ __launch_bounds__(256) void bp_batch_kernel(const BpArgs *__restrict_
             item = it;
         }
         __syncthreads();
-        const int it = item;
+        // uniform: the item's and the stack's fields stay in scalar registers
+        const int it = __builtin_amdgcn_readfirstlane(item);
         __syncthreads();
         if (it < 0) break;
         const int4 w = items[it];
+        if (flags && !flags[w.x]) continue;
         const BpArgs a = stacks[w.x];
         bp_lds_tile<ZT, INTERP, EXACT, KC, ((ZT == 32 && KC == 4) || (ZT == 16 && KC == 8)) ? 1 : 0>(
             a, w.y, w.z, w.w, sm, sb0);
@@ -664,11 +674,12 @@ __global__ __launch_bounds__(256) void bp_batch_kernel(const BpArgs *__restrict_
     }
 }
 
-// Clears the eight partition counters (a kernel, not a memset, so that the
-// launch sequence can be captured in a graph).
+// Clears the partition counters of the (at most three) persistent launches
+// (a kernel, not a memset, so that the launch sequence can be captured in a
+// graph).
 __global__ void reset_counter_kernel(int *counter)
 {
-    if (threadIdx.x < 8) counter[threadIdx.x] = 0;
+    if (threadIdx.x < 24) counter[threadIdx.x] = 0;
 }
 
 template <int ZT, int INTERP>
@@ -1226,7 +1237,20 @@ struct mr_bp_plan {
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     int tilt = 0;                         // BpArgs::tilt branch (0: no tilt correction)
     size_t tilt_row0 = 0;                 // first detector row of the next block
+    // matrix-core form (fused): scale per slice | partial maxima | flag
+    void *d_split = nullptr;
+    size_t split_cap = 0;                 // bytes
+    bool no_split = false;                // the split samples did not fit the memory: VALU kernel
 };
+
+namespace mr {
+// whether a plan with nk used projections runs on the matrix cores
+static bool plan_bpm(const mr_bp_plan *p, size_t nk, int &tile)
+{
+    return p->p.fused && p->p.interp == MR_INTERP_LINEAR && p->impl == 1 && p->tilt == 0 && !p->stage64 && !p->no_split &&
+           bpm_shape((int)p->p.width, (int)p->p.slices, (int)nk, tile);
+}
+}  // namespace mr
 
 namespace {
 
@@ -1246,17 +1270,39 @@ inline TableLayout table_layout(size_t nt, size_t n_proj)
 
 int ensure_capacity(mr_bp_plan *p, size_t n_proj, size_t n_used)
 {
-    const size_t need = std::max<size_t>(n_used, 1) * p->p.width * p->vpad;
-    const size_t nt = std::max<size_t>(n_used, 1);
+    size_t need = std::max<size_t>(n_used, 1) * p->p.width * p->vpad;
+    const size_t need_f32 = need, nt = std::max<size_t>(n_used, 1);
+    size_t split_bytes = 0;
+    int tile;
+    if (mr::plan_bpm(p, n_used, tile)) {
+        // the split samples, or the float ones when they do not fit the split
+        need = std::max(need, n_used * 2 * (size_t)mr::bpm_npair((int)p->p.width) * (size_t)mr::bpm_vp((int)p->p.slices));
+        split_bytes = sizeof(float2) * p->p.slices + sizeof(unsigned) * (mr::bpm_part_words(p->p.slices, n_used) + 1);
+    }
     const TableLayout tl = table_layout(nt, std::max<size_t>(n_proj, 1));
     // a buffer about to be replaced may still be read by the last call's kernels
-    if (p->done_ev && (need > p->sino_cap || tl.bytes > p->tables_cap))
+    if (p->done_ev && (need > p->sino_cap || tl.bytes > p->tables_cap || split_bytes > p->split_cap))
         MR_HIP(hipEventSynchronize(p->done_ev));
+    if (split_bytes > p->split_cap) {
+        if (p->d_split) (void)hipFree(p->d_split);
+        p->d_split = nullptr;
+        p->split_cap = 0;
+        MR_HIP(hipMalloc(&p->d_split, split_bytes));
+        p->split_cap = split_bytes;
+    }
     if (need > p->sino_cap) {
         if (p->d_sino) (void)hipFree(p->d_sino);
         p->d_sino = nullptr;
         p->sino_cap = 0;
-        MR_HIP(hipMalloc(&p->d_sino, need * sizeof(float)));
+        hipError_t e = hipMalloc(&p->d_sino, need * sizeof(float));
+        if (e != hipSuccess && need > need_f32) {
+            // no room for the split samples: the float sinogram may still fit
+            (void)hipGetLastError();
+            p->no_split = true;
+            need = need_f32;
+            e = hipMalloc(&p->d_sino, need * sizeof(float));
+        }
+        if (e != hipSuccess) return mr::hip_fail(e, "hipMalloc(sinogram)", __FILE__, __LINE__);
         p->sino_cap = need;
     }
     if (tl.bytes > p->tables_cap) {
@@ -1336,6 +1382,7 @@ extern "C" int mr_bp_plan_destroy(mr_bp_plan *plan)
     if (plan->d_sino) (void)hipFree(plan->d_sino);
     if (plan->d_tables) (void)hipFree(plan->d_tables);
     if (plan->d_adj) (void)hipFree(plan->d_adj);
+    if (plan->d_split) (void)hipFree(plan->d_split);
     if (plan->stage_ev) {
         (void)hipEventSynchronize(plan->stage_ev);
         (void)hipEventDestroy(plan->stage_ev);
@@ -1356,8 +1403,12 @@ extern "C" int mr_bp_plan_kernel(const mr_bp_plan *plan, char *name, size_t len)
     MR_GUARD_BEGIN
     mr::clear_error();
     MR_REQUIRE(plan != nullptr && name != nullptr && len > 0, "NULL argument");
-    const std::string d = mr::describe_bp((int)plan->p.width, (int)plan->p.slices, plan->p.interp, plan->impl,
-                                          plan->p.fused ? 0 : 1, plan->tilt);
+    int tile = 0;
+    // with tables loaded, the form their projection count selects
+    const std::string d = plan->loaded && mr::plan_bpm(plan, plan->loaded_nk, tile)
+                              ? "bp_mfma_kernel tile=" + std::to_string(tile)
+                              : mr::describe_bp((int)plan->p.width, (int)plan->p.slices, plan->p.interp, plan->impl,
+                                                plan->p.fused ? 0 : 1, plan->tilt);
     std::snprintf(name, len, "%s", d.c_str());
     return MR_OK;
     MR_GUARD_END
@@ -1429,7 +1480,25 @@ int bp_enqueue(mr_bp_plan *plan, const float *d_proj, float *d_volume, int accum
     const mr_bp_params &q = plan->p;
     const size_t nk = plan->loaded_nk;
     MR_REQUIRE(nk == 0 || d_proj != nullptr, "NULL projection pointer");
-    if (nk > 0) {
+    int tile = 0;
+    // accumulation onto a volume keeps the VALU kernel, whose running sum
+    // starts from the volume
+    const bool bpm = !accumulate && plan_bpm(plan, nk, tile);
+    int *flag = nullptr;
+    if (bpm) {
+        mr::BpmArgs m{};
+        float2 *scale = static_cast<float2 *>(plan->d_split);
+        unsigned *part = reinterpret_cast<unsigned *>(scale + q.slices);
+        flag = reinterpret_cast<int *>(part + mr::bpm_part_words(q.slices, nk));
+        m.split = reinterpret_cast<const unsigned *>(plan->d_sino);
+        m.vol = d_volume; m.tab = plan->d_tab; m.mask = plan->d_mask; m.scale = scale; m.flag = flag;
+        m.nu = (int)q.width; m.nv = (int)q.slices; m.vp = mr::bpm_vp(m.nv); m.npair = mr::bpm_npair(m.nu);
+        m.nk = (int)nk; m.nz4 = (int)((q.slices / 4) * 4);
+        int rc = mr::launch_bp_scale(d_proj, plan->d_idx, plan->d_w, m.nu, m.nv, m.nk, part, scale, flag, s);
+        if (rc == MR_OK) rc = mr::launch_bp_split_prep(m, d_proj, plan->d_idx, plan->d_w, (int)plan->vpad, s);
+        if (rc == MR_OK) rc = mr::run_bpm(m, tile, s);
+        if (rc != MR_OK) return rc;
+    } else if (nk > 0) {
         const int rc = mr::launch_bp_prep(d_proj, plan->d_sino, plan->d_idx, plan->d_w, (int)q.width,
                                           (int)q.slices, (int)plan->vpad, (int)nk, s);
         if (rc != MR_OK) return rc;
@@ -1441,6 +1510,7 @@ int bp_enqueue(mr_bp_plan *plan, const float *d_proj, float *d_volume, int accum
     a.bstride = q.multiprojbp ? a.nz4 : (int)plan->vpad;
     a.accumulate = accumulate ? 1 : 0;
     a.stage64 = plan->stage64;
+    a.gate = flag;
     a.tilt = plan->tilt;
     if (plan->tilt) mr::bp_tilt_terms(q.tilt_angle, q.tilt_pivot, plan->tilt_row0, a.tilt_co, a.tilt_ci);
     return mr::run_bp(a, q.interp, plan->impl, q.fused ? 0 : 1, s);
@@ -1696,6 +1766,12 @@ struct BatchStack {
     float *d_w = nullptr;
     size_t vpad = 0, n_used = 0;
     mr::BpArgs args{};
+    // matrix-core form (fused batches): scale per slice | partial maxima
+    bool bpm = false;
+    int tile = 0;
+    float2 *d_scale = nullptr;
+    unsigned *d_part = nullptr;
+    mr::BpmArgs margs{};
 };
 
 struct Variant {
@@ -1708,16 +1784,28 @@ inline int zt_list(int zt) { return zt == 32 ? 0 : 1; }
 
 }  // namespace
 
+// Work items of one persistent launch: int4 items and nine partition
+// boundaries, on the device.
+struct ItemList {
+    int4 *d_items = nullptr;
+    int *d_parts = nullptr;
+    int n = 0;
+};
+
 struct mr_batch_plan {
     std::vector<BatchStack> stacks;
     mr::BpArgs *d_args = nullptr;
-    int4 *d_items[2] = {nullptr, nullptr};   // item lists for ZT = 32 and ZT = 16
-    int *d_parts[2] = {nullptr, nullptr};    // 9 partition boundaries per list
-    int n_items[2] = {0, 0};
-    int *d_counter = nullptr;                // 8 partition counters
+    // VALU items for ZT = 32 and ZT = 16: [0] of the stacks that always run
+    // there, [1] of the others, for when their samples do not fit the split
+    ItemList valu[2][2];
+    ItemList mfma;                           // items of the matrix-core kernel
+    mr::BpmArgs *d_margs = nullptr;
+    int *d_flags = nullptr;                  // per stack: samples do not fit the split
+    int *d_counter = nullptr;                // 8 partition counters per launch
     int variant = 0;
     int exact = 1;                           // 0: interpolation folded into FMAs (MR_BATCH_FUSED)
     int grid[kNumVariants] = {0};
+    int mfma_grid = 0;
     double updates = 0.0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -1726,22 +1814,21 @@ struct mr_batch_plan {
 
 namespace {
 
-int batch_launch_bp(mr_batch_plan *p, int variant, hipStream_t s)
+// The VALU kernel over one list.
+int batch_launch_valu(mr_batch_plan *p, int variant, const ItemList &l, int *counter, const int *flags, hipStream_t s)
 {
+    if (l.n == 0) return MR_OK;
     const Variant v = kVariants[variant];
-    const int li = zt_list(v.zt);
-    hipLaunchKernelGGL(mr::reset_counter_kernel, dim3(1), dim3(64), 0, s, p->d_counter);
-    MR_HIP(hipGetLastError());
-    mr::ProfScope prof("bp_batch", s);
     dim3 grid((unsigned)p->grid[variant]), block(256);
+    const int ns = (int)p->stacks.size();
 #define MR_BATCH_CASE(ZT, KC)                                                                         \
     if (v.zt == ZT && v.kc == KC) {                                                                   \
         if (p->exact)                                                                                 \
             hipLaunchKernelGGL((mr::bp_batch_kernel<ZT, 0, true, KC>), grid, block, 0, s, p->d_args,   \
-                               p->d_items[li], p->d_parts[li], p->d_counter);                         \
+                               l.d_items, l.d_parts, counter, flags, ns);                             \
         else                                                                                          \
             hipLaunchKernelGGL((mr::bp_batch_kernel<ZT, 0, false, KC>), grid, block, 0, s, p->d_args,  \
-                               p->d_items[li], p->d_parts[li], p->d_counter);                         \
+                               l.d_items, l.d_parts, counter, flags, ns);                             \
     }
     MR_BATCH_CASE(32, 4)
     MR_BATCH_CASE(32, 8)
@@ -1753,6 +1840,20 @@ int batch_launch_bp(mr_batch_plan *p, int variant, hipStream_t s)
     return MR_OK;
 }
 
+int batch_launch_bp(mr_batch_plan *p, int variant, hipStream_t s)
+{
+    const int li = zt_list(kVariants[variant].zt);
+    hipLaunchKernelGGL(mr::reset_counter_kernel, dim3(1), dim3(64), 0, s, p->d_counter);
+    MR_HIP(hipGetLastError());
+    mr::ProfScope prof("bp_batch", s);
+    int rc = MR_OK;
+    if (p->mfma.n > 0)
+        rc = mr::launch_bpm_batch(p->d_margs, p->mfma.d_items, p->mfma.d_parts, p->d_counter, p->mfma_grid, s);
+    if (rc == MR_OK) rc = batch_launch_valu(p, variant, p->valu[0][li], p->d_counter + 8, nullptr, s);
+    if (rc == MR_OK) rc = batch_launch_valu(p, variant, p->valu[1][li], p->d_counter + 16, p->d_flags, s);
+    return rc;
+}
+
 int batch_prepare(mr_batch_plan *p, hipStream_t s)
 {
     for (auto &b : p->stacks) {
@@ -1760,6 +1861,13 @@ int batch_prepare(mr_batch_plan *p, hipStream_t s)
         int rc = mr::filter_rows_to(b.fplan, d.d_proj, b.d_filt, d.n_proj * d.slices, s);
         if (rc != MR_OK) return rc;
         if (b.n_used == 0) continue;
+        if (b.bpm) {
+            rc = mr::launch_bp_scale(b.d_filt, b.d_idx, b.d_w, b.margs.nu, b.margs.nv, b.margs.nk, b.d_part, b.d_scale,
+                                     const_cast<int *>(b.margs.flag), s);
+            if (rc == MR_OK) rc = mr::launch_bp_split_prep(b.margs, b.d_filt, b.d_idx, b.d_w, (int)b.vpad, s);
+            if (rc != MR_OK) return rc;
+            continue;
+        }
         rc = mr::launch_bp_prep(b.d_filt, b.d_sino, b.d_idx, b.d_w, (int)d.width, (int)d.slices, (int)b.vpad,
                                 (int)b.n_used, s);
         if (rc != MR_OK) return rc;
@@ -1774,13 +1882,41 @@ void batch_free(mr_batch_plan *p)
     for (auto &b : p->stacks) {
         if (b.fplan) mr_filter_plan_destroy(b.fplan);
         for (void *ptr : {(void *)b.d_filt, (void *)b.d_sino, (void *)b.d_tab, (void *)b.d_mask,
-                          (void *)b.d_idx, (void *)b.d_w})
+                          (void *)b.d_idx, (void *)b.d_w, (void *)b.d_scale, (void *)b.d_part})
             if (ptr) (void)hipFree(ptr);
     }
-    for (void *ptr : {(void *)p->d_args, (void *)p->d_items[0], (void *)p->d_items[1], (void *)p->d_parts[0],
-                      (void *)p->d_parts[1], (void *)p->d_counter})
+    for (ItemList *l : {&p->valu[0][0], &p->valu[0][1], &p->valu[1][0], &p->valu[1][1], &p->mfma}) {
+        if (l->d_items) (void)hipFree(l->d_items);
+        if (l->d_parts) (void)hipFree(l->d_parts);
+    }
+    for (void *ptr : {(void *)p->d_args, (void *)p->d_margs, (void *)p->d_flags, (void *)p->d_counter})
         if (ptr) (void)hipFree(ptr);
     delete p;
+}
+
+// Uploads items (cost, item) in spatial order, cut into eight contiguous
+// partitions of equal cost, one per XCD.
+hipError_t upload_items(const std::vector<std::pair<double, int4>> &v, ItemList &l)
+{
+    if (v.empty()) return hipSuccess;
+    double total = 0;
+    for (const auto &it : v) total += it.first;
+    std::vector<int> parts(9, (int)v.size());
+    parts[0] = 0;
+    double acc = 0;
+    int next = 1;
+    for (size_t k = 0; k < v.size() && next < 8; ++k) {
+        acc += v[k].first;
+        while (next < 8 && acc >= total * next / 8.0) parts[next++] = (int)k + 1;
+    }
+    std::vector<int4> flat(v.size());
+    for (size_t k = 0; k < v.size(); ++k) flat[k] = v[k].second;
+    l.n = (int)flat.size();
+    hipError_t e = hipMalloc(&l.d_items, sizeof(int4) * flat.size());
+    if (e == hipSuccess) e = hipMemcpy(l.d_items, flat.data(), sizeof(int4) * flat.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMalloc(&l.d_parts, sizeof(int) * 9);
+    if (e == hipSuccess) e = hipMemcpy(l.d_parts, parts.data(), sizeof(int) * 9, hipMemcpyHostToDevice);
+    return e;
 }
 
 template <int ZT, int KC>
@@ -1811,7 +1947,11 @@ extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *
     auto *p = new mr_batch_plan();
     p->exact = (flags & MR_BATCH_FUSED) ? 0 : 1;
     p->stacks.resize(n_stacks);
-    std::vector<std::pair<double, int4>> items[2];   // ZT = 32, ZT = 16
+    std::vector<std::pair<double, int4>> items[2][2], mitems;   // [matrix-core stack][ZT = 32, ZT = 16]
+    if (hipError_t e = hipMalloc(&p->d_flags, sizeof(int) * n_stacks); e != hipSuccess) {
+        batch_free(p);
+        return mr::hip_fail(e, "mr_batch_plan_create flags", __FILE__, __LINE__);
+    }
     for (size_t i = 0; i < n_stacks; ++i) {
         BatchStack &b = p->stacks[i];
         b.desc = stacks[i];
@@ -1842,8 +1982,15 @@ extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *
             m[y].x = (int)first[y];
             m[y].y = (int)std::max(first[y], second[y]);
         }
+        b.bpm = !p->exact && mr::bpm_shape((int)d.width, (int)d.slices, (int)b.n_used, b.tile);
+        size_t sino = std::max<size_t>(b.n_used, 1) * d.width * b.vpad;
+        if (b.bpm)
+            sino = std::max(sino, b.n_used * 2 * (size_t)mr::bpm_npair((int)d.width) * mr::bpm_vp((int)d.slices));
         hipError_t e = hipMalloc(&b.d_filt, sizeof(float) * d.n_proj * d.slices * d.width);
-        if (e == hipSuccess) e = hipMalloc(&b.d_sino, sizeof(float) * std::max<size_t>(b.n_used, 1) * d.width * b.vpad);
+        if (e == hipSuccess) e = hipMalloc(&b.d_sino, sizeof(float) * sino);
+        if (e == hipSuccess && b.bpm) e = hipMalloc(&b.d_scale, sizeof(float2) * d.slices);
+        if (e == hipSuccess && b.bpm)
+            e = hipMalloc(&b.d_part, sizeof(unsigned) * mr::bpm_part_words(d.slices, b.n_used));
         if (e == hipSuccess) e = hipMalloc(&b.d_tab, sizeof(float4) * std::max<size_t>(b.n_used, 1));
         if (e == hipSuccess) e = hipMalloc(&b.d_mask, sizeof(int2) * d.width);
         if (e == hipSuccess) e = hipMalloc(&b.d_idx, sizeof(int) * std::max<size_t>(b.n_used, 1));
@@ -1862,13 +2009,19 @@ extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *
         a.sino = b.d_sino; a.vol = d.d_volume; a.tab = b.d_tab; a.mask = b.d_mask;
         a.nu = (int)d.width; a.nv = (int)d.slices; a.vpad = (int)b.vpad; a.nk = (int)b.n_used;
         a.nz4 = (int)((d.slices / 4) * 4); a.bstride = (int)b.vpad; a.accumulate = 0;
+        if (b.bpm) {
+            mr::BpmArgs &q = b.margs;
+            q.split = reinterpret_cast<const unsigned *>(b.d_sino);
+            q.vol = d.d_volume; q.tab = b.d_tab; q.mask = b.d_mask; q.scale = b.d_scale; q.flag = p->d_flags + i;
+            q.nu = a.nu; q.nv = a.nv; q.vp = mr::bpm_vp(a.nv); q.npair = mr::bpm_npair(a.nu);
+            q.nk = a.nk; q.nz4 = a.nz4;
+            a.gate = q.flag;   // the single-stack launch behind the matrix-core one
+        }
         p->updates += (double)d.width * d.width * d.slices * d.n_proj;
         // work items in spatial order (slice chunk, stripes of 4 tile
         // columns, rows, columns), cost ~ projections x voxels inside the circle
         const int tiles = (int)((d.width + 15) / 16);
-        for (int li = 0; li < 2; ++li) {
-            const int ZT = li == 0 ? 32 : 16;
-            const int zc = (int)((d.slices + ZT - 1) / ZT);
+        auto spatial = [&](int zc, auto &&emit) {
             for (int bz = 0; bz < zc; ++bz)
                 for (int sx = 0; sx < tiles; sx += 4)
                     for (int by = 0; by < tiles; ++by)
@@ -1878,32 +2031,31 @@ extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *
                                 const int lo = std::max(m[yy].x, bx * 16), hi = std::min(m[yy].y, bx * 16 + 16);
                                 inside += std::max(0, hi - lo);
                             }
-                            const double cost = 1.0 + inside * (double)b.n_used * std::min<int>(ZT, (int)d.slices - bz * ZT);
-                            items[li].push_back({cost, make_int4((int)i, bx, by, bz)});
+                            emit(bx, by, bz, inside * (double)b.n_used);
                         }
+        };
+        for (int li = 0; li < 2; ++li) {
+            const int ZT = li == 0 ? 32 : 16;
+            spatial((int)((d.slices + ZT - 1) / ZT), [&](int bx, int by, int bz, double work) {
+                items[b.bpm ? 1 : 0][li].push_back({1.0 + work * std::min<int>(ZT, (int)d.slices - bz * ZT),
+                                                    make_int4((int)i, bx, by, bz)});
+            });
+        }
+        if (b.bpm) {
+            // chunks of four slice tiles, the rest in one of its own (as
+            // run_bpm); a chunk costs about 1.5 tiles beside its own
+            const int nzt = mr::bpm_vp((int)d.slices) / 16;
+            spatial((nzt + 3) / 4, [&](int bx, int by, int bz, double work) {
+                const int nt = std::min(4, nzt - 4 * bz);
+                mitems.push_back({1.0 + work * (1.5 + nt), make_int4((int)i, bx, by, 4 * bz | nt << 16)});
+            });
         }
     }
-    for (int li = 0; li < 2; ++li) {
-        // eight contiguous partitions of equal cost, one per XCD
-        const auto &v = items[li];
-        double total = 0;
-        for (const auto &it : v) total += it.first;
-        std::vector<int> parts(9, (int)v.size());
-        parts[0] = 0;
-        double acc = 0;
-        int next = 1;
-        for (size_t k = 0; k < v.size() && next < 8; ++k) {
-            acc += v[k].first;
-            while (next < 8 && acc >= total * next / 8.0) parts[next++] = (int)k + 1;
-        }
-        std::vector<int4> flat(v.size());
-        for (size_t k = 0; k < v.size(); ++k) flat[k] = v[k].second;
-        p->n_items[li] = (int)flat.size();
-        hipError_t e = hipMalloc(&p->d_items[li], sizeof(int4) * std::max<size_t>(flat.size(), 1));
-        if (e == hipSuccess && !flat.empty())
-            e = hipMemcpy(p->d_items[li], flat.data(), sizeof(int4) * flat.size(), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMalloc(&p->d_parts[li], sizeof(int) * 9);
-        if (e == hipSuccess) e = hipMemcpy(p->d_parts[li], parts.data(), sizeof(int) * 9, hipMemcpyHostToDevice);
+    {
+        hipError_t e = upload_items(mitems, p->mfma);
+        for (int k = 0; k < 2; ++k)
+            for (int li = 0; li < 2; ++li)
+                if (e == hipSuccess) e = upload_items(items[k][li], p->valu[k][li]);
         if (e != hipSuccess) {
             batch_free(p);
             return mr::hip_fail(e, "mr_batch_plan_create items", __FILE__, __LINE__);
@@ -1913,7 +2065,12 @@ extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *
     for (size_t i = 0; i < n_stacks; ++i) args[i] = p->stacks[i].args;
     hipError_t e = hipMalloc(&p->d_args, sizeof(mr::BpArgs) * n_stacks);
     if (e == hipSuccess) e = hipMemcpy(p->d_args, args.data(), sizeof(mr::BpArgs) * n_stacks, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMalloc(&p->d_counter, sizeof(int) * 8);
+    std::vector<mr::BpmArgs> margs(n_stacks);
+    for (size_t i = 0; i < n_stacks; ++i) margs[i] = p->stacks[i].margs;
+    if (e == hipSuccess) e = hipMalloc(&p->d_margs, sizeof(mr::BpmArgs) * n_stacks);
+    if (e == hipSuccess)
+        e = hipMemcpy(p->d_margs, margs.data(), sizeof(mr::BpmArgs) * n_stacks, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMalloc(&p->d_counter, sizeof(int) * 24);
     if (e != hipSuccess) {
         batch_free(p);
         return mr::hip_fail(e, "mr_batch_plan_create args", __FILE__, __LINE__);
@@ -1924,6 +2081,7 @@ extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *
     if (rc == MR_OK) rc = occupancy_grid<16, 8>(p->grid[2], p->exact);
     if (rc == MR_OK) rc = occupancy_grid<16, 4>(p->grid[3], p->exact);
     if (rc == MR_OK) rc = occupancy_grid<16, 16>(p->grid[4], p->exact);
+    if (rc == MR_OK && p->mfma.n > 0) rc = mr::bpm_batch_grid(p->mfma_grid);
     if (rc != MR_OK) {
         batch_free(p);
         return rc;
@@ -1970,9 +2128,12 @@ extern "C" int mr_batch_plan_info(const mr_batch_plan *plan, int *slice_tile, in
     mr::clear_error();
     MR_REQUIRE(plan != nullptr, "plan is NULL");
     const Variant v = kVariants[plan->variant];
-    if (slice_tile) *slice_tile = v.zt;
-    if (proj_chunk) *proj_chunk = v.kc;
-    if (n_items) *n_items = (size_t)plan->n_items[zt_list(v.zt)];
+    const ItemList &l = plan->valu[0][zt_list(v.zt)];
+    // the matrix-core kernel's shape when every stack runs there
+    const bool all_mfma = l.n == 0 && plan->mfma.n > 0;
+    if (slice_tile) *slice_tile = all_mfma ? 64 : v.zt;
+    if (proj_chunk) *proj_chunk = all_mfma ? 4 : v.kc;
+    if (n_items) *n_items = (size_t)l.n + (size_t)plan->mfma.n;
     if (updates) *updates = plan->updates;
     return MR_OK;
     MR_GUARD_END
@@ -2026,7 +2187,8 @@ extern "C" int mr_batch_run_sequential(mr_batch_plan *plan, void *stream)
     int rc = batch_prepare(plan, s);
     if (rc != MR_OK) return rc;
     for (auto &b : plan->stacks) {
-        rc = mr::run_bp(b.args, 0, 1, plan->exact, s);
+        if (b.bpm) rc = mr::run_bpm(b.margs, b.tile, s);
+        if (rc == MR_OK) rc = mr::run_bp(b.args, 0, 1, plan->exact, s);
         if (rc != MR_OK) return rc;
     }
     return MR_OK;

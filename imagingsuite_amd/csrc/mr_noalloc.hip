@@ -8,16 +8,21 @@
 //
 //   scratch layout (bytes)
 //     [0, kTableBytes)             mask int2[width] | tab float4[n_used] |
-//                                  idx int[n_used] | w float[n_proj], each
-//                                  part 256-byte aligned
-//     [kTableBytes, kScratchBytes) sinogram chunk [kc][width][vpad]
+//                                  idx int[n_used] | w float[n_proj] | scale
+//                                  float2[slices] | flag, each part 256-byte
+//                                  aligned (the last two: matrix-core form)
+//     [kTableBytes, kScratchBytes) sinogram chunk [kc][width][vpad], or its
+//                                  split samples (mr_bp_mfma.hip)
 //
 // The used projections are back-projected in chunks of kc = as many staged
 // projections as fit; each chunk is weighted/transposed into the scratch and
 // added to the volume by the same kernels as mr_bp_parallel.  Every voxel
 // still accumulates the projections one after the other in the reference's
 // order (the kernels load the voxel, add the chunk's projections in order
-// and store it), so the result equals mr_bp_parallel's bit for bit.
+// and store it), so the result equals mr_bp_parallel's bit for bit.  In the
+// matrix-core form the samples' scale comes from all projections before the
+// first chunk, chunks are whole groups of four projections and a chunk
+// continues the sums of the ones before it: the same bits again.
 //
 // The host tables reach the scratch through kernel arguments (scratch_put_kernel),
 // so no host buffer has to outlive the call and nothing is allocated.
@@ -39,7 +44,7 @@
 namespace {
 
 constexpr size_t kScratchBytes = MR_NOALLOC_SCRATCH_BYTES;
-constexpr size_t kTableBytes = size_t(4) << 20;   // mask + tables (at most about 2.3 MiB)
+constexpr size_t kTableBytes = size_t(4) << 20;   // mask + tables (at most about 2.8 MiB)
 constexpr int kMaxDevices = 64;
 constexpr unsigned kPutWords = 480;               // words per scratch_put_kernel launch (1.9 KB of arguments)
 
@@ -117,7 +122,9 @@ extern "C" int mr_bp_parallel_noalloc(const mr_bp_params *params, const float *d
     const size_t off_idx = off_tab + align256(sizeof(float4) * nk);
     const size_t off_w = off_idx + align256(sizeof(int) * nk);
     const size_t table_end = off_w + sizeof(float) * n_proj;
-    MR_REQUIRE(table_end <= kTableBytes, "tables exceed the fixed scratch");   // cannot happen with the limits above
+    const size_t off_scale = align256(table_end), off_flag = off_scale + align256(sizeof(float2) * q.slices);
+    MR_REQUIRE(off_flag + sizeof(int) <= kTableBytes &&
+               table_end <= kTableBytes, "tables exceed the fixed scratch");   // cannot happen with the limits above
 
     int dev = 0;
     MR_HIP(hipGetDevice(&dev));
@@ -165,7 +172,26 @@ extern "C" int mr_bp_parallel_noalloc(const mr_bp_params *params, const float *d
     const int *d_idx = reinterpret_cast<const int *>(base + off_idx);
     const float *d_w = reinterpret_cast<const float *>(base + off_w);
     float *d_sino = reinterpret_cast<float *>(base + kTableBytes);
-    const size_t kc_max = sino_bytes / proj_bytes;
+    const int impl = (q.multiprojbp && (q.slices & 3)) ? 0 : 1;
+    int tile = 0;
+    const bool bpm = q.fused && !accumulate && q.interp == MR_INTERP_LINEAR && impl == 1 &&
+                     mr::bpm_shape((int)q.width, (int)q.slices, (int)nk, tile);
+    mr::BpmArgs m{};
+    size_t kc_max = sino_bytes / proj_bytes;
+    if (bpm) {
+        float2 *scale = reinterpret_cast<float2 *>(base + off_scale);
+        int *flag = reinterpret_cast<int *>(base + off_flag);
+        m.split = reinterpret_cast<const unsigned *>(d_sino);
+        m.vol = d_volume; m.mask = d_mask; m.scale = scale; m.flag = flag;
+        m.nu = (int)q.width; m.nv = (int)q.slices; m.vp = mr::bpm_vp(m.nv); m.npair = mr::bpm_npair(m.nu);
+        m.nz4 = (int)((q.slices / 4) * 4);
+        // groups of four that fit as split or as float samples (at least one: bpm_shape)
+        kc_max = std::min(kc_max, sino_bytes / (8 * (size_t)m.npair * (size_t)m.vp)) / 4 * 4;
+        MR_REQUIRE(mr::bpm_part_words(q.slices, nk) * sizeof(unsigned) <= sino_bytes, "slices exceed the fixed scratch");
+        rc = mr::launch_bp_scale(d_proj, d_idx, d_w, m.nu, m.nv, (int)nk, reinterpret_cast<unsigned *>(d_sino), scale,
+                                 flag, s);
+        if (rc != MR_OK) return rc;
+    }
 
     mr::BpArgs a{};
     a.vol = d_volume;
@@ -176,12 +202,19 @@ extern "C" int mr_bp_parallel_noalloc(const mr_bp_params *params, const float *d
     a.vpad = (int)vpad;
     a.nz4 = (int)((q.slices / 4) * 4);
     a.bstride = q.multiprojbp ? a.nz4 : (int)vpad;
-    const int impl = (q.multiprojbp && (q.slices & 3)) ? 0 : 1;
+    a.gate = m.flag;
     // nk == 0 still runs one launch: it writes the zeroed (or unchanged) volume
     size_t kb = 0;
     do {
         const size_t kc = std::min(kc_max, nk - kb);
-        if (kc > 0) {
+        if (bpm) {
+            m.tab = d_tab + kb;
+            m.nk = (int)kc;
+            m.chain = kb > 0 ? 1 : 0;
+            rc = mr::launch_bp_split_prep(m, d_proj, d_idx + kb, d_w, (int)vpad, s);
+            if (rc == MR_OK) rc = mr::run_bpm(m, tile, s);
+            if (rc != MR_OK) return rc;
+        } else if (kc > 0) {
             rc = mr::launch_bp_prep(d_proj, d_sino, d_idx + kb, d_w, (int)q.width, (int)q.slices, (int)vpad,
                                     (int)kc, s);
             if (rc != MR_OK) return rc;
