@@ -12,11 +12,19 @@ namespace mr {
 // p = img - dark (or img); p <= 0 ? 0 : flat_log - log(p) + dl (no flat:
 // -log(p) + dl).  Shared by the normalisation kernel and the filter's fused
 // load, so that both give the same values.
+__device__ __forceinline__ float lognorm_value(float v, bool has_flat, float flat_log, bool has_dark, float dark,
+                                               float dl)
+{
+    const float p = has_dark ? v - dark : v;
+    const float l = logf(p);
+    const float r = (has_flat ? flat_log - l : -l) + dl;
+    return p <= 0.0f ? 0.0f : r;
+}
+
 __device__ __forceinline__ float lognorm_px(float v, const float *flat_log, const float *dark, size_t i, float dl)
 {
-    const float p = dark ? v - dark[i] : v;
-    if (p <= 0.0f) return 0.0f;
-    return flat_log ? flat_log[i] - logf(p) + dl : -logf(p) + dl;
+    return lognorm_value(v, flat_log != nullptr, flat_log ? flat_log[i] : 0.0f, dark != nullptr, dark ? dark[i] : 0.0f,
+                         dl);
 }
 
 struct RowFilterArgs {
@@ -29,8 +37,8 @@ struct RowFilterArgs {
                                 // mode 3
     int insert;                 // mode 0: nInsert; mode 1: (P - n) / 2
     const float *taper;         // mode 0: nInsert sigmoid weights
-    const float *hs;            // P real spectral multipliers
-    const float2 *tw;           // P twiddles exp(-2 pi i k / P)
+    const float *hs;            // P real spectral multipliers (spectrum_order)
+    const float2 *tw;           // the stages' twiddles (make_twiddles)
     float post0, post1, post2;  // sequential output multipliers
     const float *pre_w;         // mode 1: per-projection input weight (nullable)
     int rows_per_proj;          // rows of one projection (mode 1)
@@ -65,6 +73,7 @@ int filter_rows_to(mr_filter_plan *plan, const float *in, float *out, size_t n_r
 size_t filter_width(const mr_filter_plan *plan);
 int run_fdk_margin_rows(float *img, int n, int h, long n_proj, hipStream_t s);
 std::vector<float> make_twiddles(size_t P);
+std::vector<float> spectrum_order(const std::vector<float> &h);
 // Zero-fills n floats with a kernel (no hipMemset, so callers may capture it in a graph).
 int fill_zero(float *d, size_t n, hipStream_t s);
 

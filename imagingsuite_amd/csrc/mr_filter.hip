@@ -63,85 +63,149 @@ __device__ __forceinline__ float fdk_row_vv2(const RowFilterArgs &a, long r)
     return vv * vv;
 }
 
-// The filter on the radix-8 padded FFT (fft_lds2): dynamic LDS holds the
-// padded line (lds_len(P) float2) followed by the P/8 twiddles it uses.
-template <int P, int NT>
-__global__ __launch_bounds__(NT) void row_filter_kernel2(RowFilterArgs a)
+// Threads of a block whose stages have NB butterflies (or more, at P = 16384):
+// one butterfly per thread; two at P = 8192, where the 1024 threads of a block
+// would have 64 registers each to keep two blocks on a CU and spill (20 000
+// rows of 4000: 308 us, 368 with one block of 1024 per CU, 515 with spills; at
+// P = 4096 two butterflies per thread take 542 us against 480).
+constexpr int filter_threads(int P, int NB) { return P == 8192 ? NB / 2 : NB; }
+
+// One row pair per block; dynamic LDS holds the line (P float2).  The padded
+// line is built in the first stage's loads and the kept samples are cropped and
+// scaled in the last stage: no LDS round trip of their own.  SHORT: modes 3 and
+// 4, whose rows (n <= P / 2 samples) fill the first half of the line.
+//
+// Bound by latency and issue together: at P = 4096 the vector ALU issues for
+// about half of the time and LDS is busy for a quarter (no bank conflicts), at
+// 8 waves per SIMD; hence all of a thread's global loads in flight at once, and
+// twiddles, spectrum and responses requested ahead of the exchange before their
+// use.  76 800 rows of 2048: 480 us (2.6 TB/s) against 676 with Stockham stages
+// (two block barriers each, the twiddles in LDS, 40 % of the LDS cycles bank
+// conflicts); with the normalisation of raw counts 625 against 885.
+template <int P, int NB, bool SHORT>
+__global__ __launch_bounds__(filter_threads(P, NB), P <= 4096 ? 8 : 4) void row_filter_kernel2(RowFilterArgs a)
 {
     extern __shared__ float2 line[];
-    float2 *twl = line + lds_len(P);
+    constexpr int NT = filter_threads(P, NB);
     const long r0 = 2 * (long)blockIdx.x;
     const bool has1 = r0 + 1 < a.n_rows;
     float *row0 = a.rows + r0 * a.n;
     float *row1 = has1 ? row0 + a.n : row0;
     const int t = threadIdx.x;
-    for (int i = t; i < P / 8; i += NT) twl[i] = a.tw[i];
     float *o0 = a.out ? a.out + r0 * a.n : row0;
     float *o1 = o0 + a.n;
-    if (a.mode != 2) {
-        // The padded line is built in the first pass's loads, the spectrum
-        // multiplied in the last forward pass and the kept samples cropped
-        // and scaled in the last inverse pass: no LDS round trip of their
-        // own.  Same values and operations as staging the line first.
-        float f0 = 0.f, l0 = 0.f, f1 = 0.f, l1 = 0.f, w0 = 1.f, w1 = 1.f, v0 = 0.f, v1 = 0.f;
-        float sa0 = 0.f, sa1 = 0.f, sb0 = 0.f, sb1 = 0.f;   // mode 4: the rows' dot products with the responses
-        // mode 3 with norm: row r is row r % rows_per_proj of projection r / rows_per_proj
-        const float *nf = a.norm_flat_log, *nd = a.norm_dark;
-        size_t pix0 = 0, pix1 = 0;
-        float dl0 = 0.f, dl1 = 0.f;
-        if (a.mode == 3 && a.norm) {
-            const long rr1 = has1 ? r0 + 1 : r0;
-            pix0 = (size_t)(r0 % a.rows_per_proj) * a.n;
-            pix1 = (size_t)(rr1 % a.rows_per_proj) * a.n;
-            dl0 = a.norm_dl ? a.norm_dl[r0 / a.rows_per_proj] : 0.0f;
-            dl1 = a.norm_dl ? a.norm_dl[rr1 / a.rows_per_proj] : 0.0f;
-        }
-        auto raw0 = [&](int i) { return a.norm ? lognorm_px(row0[i], nf, nd, pix0 + i, dl0) : row0[i]; };
-        auto raw1 = [&](int i) { return a.norm ? lognorm_px(row1[i], nf, nd, pix1 + i, dl1) : row1[i]; };
+    constexpr int B = P / 8, PER = (B + NT - 1) / NT;
+    auto nothing = [] {};
+    auto nothing2 = [](int, int) {};
+    // point by point: load(i) -> value, store(i, value)
+    auto each = [](auto &load) {
+        return [&load](int j, float2 (&v)[8]) {
+#pragma unroll
+            for (int r = 0; r < (SHORT ? 4 : 8); ++r) v[r] = load(j + r * B);
+        };
+    };
+    auto to_each = [](auto &store) {
+        return [&store](int, int j, const float2 (&v)[8]) {
+#pragma unroll
+            for (int r = 0; r < (SHORT ? 4 : 8); ++r) store(j + r * B, v[r]);
+        };
+    };
+    if constexpr (SHORT) {
         if (a.mode == 3) {
-            f0 = raw0(0); l0 = raw0(a.n - 1);
-            f1 = raw1(0); l1 = raw1(a.n - 1);
-        } else if (a.mode == 0) {
-            f0 = row0[0]; l0 = row0[a.n - 1];
-            f1 = row1[0]; l1 = row1[a.n - 1];
-        } else {
-            w0 = a.pre_w ? a.pre_w[r0 / a.rows_per_proj] : 1.0f;
-            w1 = (a.pre_w && has1) ? a.pre_w[(r0 + 1) / a.rows_per_proj] : 1.0f;
-            v0 = fdk_row_vv2(a, r0);
-            v1 = fdk_row_vv2(a, r0 + 1);
+            // with norm: row r is row r % rows_per_proj of projection r / rows_per_proj
+            const float *nf = a.norm_flat_log, *nd = a.norm_dark;
+            const bool norm = a.norm, flat = nf != nullptr, dark = nd != nullptr;
+            size_t pix0 = 0, pix1 = 0;
+            float dl0 = 0.f, dl1 = 0.f;
+            if (norm) {
+                const long rr1 = has1 ? r0 + 1 : r0;
+                pix0 = (size_t)(r0 % a.rows_per_proj) * a.n;
+                pix1 = (size_t)(rr1 % a.rows_per_proj) * a.n;
+                dl0 = a.norm_dl ? a.norm_dl[r0 / a.rows_per_proj] : 0.0f;
+                dl1 = a.norm_dl ? a.norm_dl[rr1 / a.rows_per_proj] : 0.0f;
+            }
+            const float *flat0 = nf + pix0, *flat1 = nf + pix1, *dark0 = nd + pix0, *dark1 = nd + pix1;
+            // the rows' ends, one per lane: first and last of row 0, of row 1
+            const int end = (t & 1) ? a.n - 1 : 0;
+            const bool second = t & 2;
+            float e = second ? row1[end] : row0[end];
+            if (norm)
+                e = lognorm_value(e, flat, flat ? (second ? flat1 : flat0)[end] : 0.0f, dark,
+                                  dark ? (second ? dark1 : dark0)[end] : 0.0f, second ? dl1 : dl0);
+            const float f0 = __shfl(e, 0), l0 = __shfl(e, 1), f1 = __shfl(e, 2), l1 = __shfl(e, 3);
+            auto load = [&](int j, float2 (&v)[8]) {
+                int i[4];
+                float x0[4], x1[4], g0[4], g1[4], d0[4], d1[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    i[r] = min(j + r * B, a.n - 1);
+                    x0[r] = row0[i[r]];
+                    x1[r] = row1[i[r]];
+                }
+                if (norm) {
+                    if (flat)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            g0[r] = flat0[i[r]];
+                            g1[r] = flat1[i[r]];
+                        }
+                    if (dark)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            d0[r] = dark0[i[r]];
+                            d1[r] = dark1[i[r]];
+                        }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        x0[r] = lognorm_value(x0[r], flat, g0[r], dark, d0[r], dl0);
+                        x1[r] = lognorm_value(x1[r], flat, g1[r], dark, d1[r], dl1);
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float s = (float)i[r] * a.ramp_inv, t1 = 1.0f - s;
+                    const bool in = j + r * B < a.n;
+                    v[r] = make_float2(in ? x0[r] - (f0 * t1 + l0 * s) : 0.0f,
+                                       in && has1 ? x1[r] - (f1 * t1 + l1 * s) : 0.0f);
+                }
+            };
+            float rf[PER][4], rl[PER][4];
+            auto before_store = [&](int q, int j) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int i = min(j + r * B, a.n - 1);
+                    rf[q][r] = a.resp_first[i];
+                    rl[q][r] = a.resp_last[i];
+                }
+            };
+            auto store = [&](int q, int j, const float2 (&v)[8]) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int i = j + r * B;
+                    if (i < a.n) {
+                        o0[i] = (v[r].x + f0 * rf[q][r]) + l0 * rl[q][r];
+                        if (has1) o1[i] = (v[r].y + f1 * rf[q][r]) + l1 * rl[q][r];
+                    }
+                }
+            };
+            fft_filter<P, NT, true>(line, a.tw, a.hs, load, nothing, before_store, store);
+            return;
         }
+        // mode 4: the rows' dot products with the responses fold back onto
+        // their ends
+        __shared__ float red[NT / 64 + 1][4];
+        float sa0 = 0.f, sa1 = 0.f, sb0 = 0.f, sb1 = 0.f;
         auto load = [&](int i) -> float2 {
-            if (a.mode == 4) {
-                if (i >= a.n) return make_float2(0.0f, 0.0f);
-                const float x0 = row0[i], x1 = has1 ? row1[i] : 0.0f;
-                const float ra = a.resp_first[i], rb = a.resp_last[i];
-                sa0 += ra * x0;
-                sa1 += ra * x1;
-                sb0 += rb * x0;
-                sb1 += rb * x1;
-                return make_float2(x0, x1);
-            }
-            if (a.mode == 3) {
-                if (i >= a.n) return make_float2(0.0f, 0.0f);
-                const float s = (float)i * a.ramp_inv, t1 = 1.0f - s;
-                return make_float2(raw0(i) - (f0 * t1 + l0 * s), has1 ? raw1(i) - (f1 * t1 + l1 * s) : 0.0f);
-            }
-            if (a.mode == 0)
-                return make_float2(pb_pad(row0, a.n, i, a.insert, P, a.taper, f0, l0),
-                                   has1 ? pb_pad(row1, a.n, i, a.insert, P, a.taper, f1, l1) : 0.0f);
-            return make_float2(fdk_pad(row0, a.n, i, a.insert, P, w0, a, v0),
-                               has1 ? fdk_pad(row1, a.n, i, a.insert, P, w1, a, v1) : 0.0f);
+            if (i >= a.n) return make_float2(0.0f, 0.0f);
+            const float x0 = row0[i], x1 = has1 ? row1[i] : 0.0f;
+            const float ra = a.resp_first[i], rb = a.resp_last[i];
+            sa0 += ra * x0;
+            sa1 += ra * x1;
+            sb0 += rb * x0;
+            sb1 += rb * x1;
+            return make_float2(x0, x1);
         };
-        auto spectrum = [&](int i, float2 v) {
-            const float h = a.hs[i];
-            line[lpad(i)] = make_float2(v.x * h, v.y * h);
-        };
-        __syncthreads();   // the twiddles
-        fft_lds2_io<P, NT, false, true, true, true>(line, twl, load, spectrum);
-        __shared__ float red4[NT / 64 + 1][4];
-        float A0 = 0.f, A1 = 0.f, B0 = 0.f, B1 = 0.f;
-        if (a.mode == 4) {
-            // block sums of the dot products, read after the barrier below
+        auto reduce = [&] {
             for (int off = 32; off > 0; off >>= 1) {
                 sa0 += __shfl_xor(sa0, off);
                 sa1 += __shfl_xor(sa1, off);
@@ -149,93 +213,71 @@ __global__ __launch_bounds__(NT) void row_filter_kernel2(RowFilterArgs a)
                 sb1 += __shfl_xor(sb1, off);
             }
             if ((t & 63) == 0) {
-                red4[t >> 6][0] = sa0;
-                red4[t >> 6][1] = sa1;
-                red4[t >> 6][2] = sb0;
-                red4[t >> 6][3] = sb1;
-            }
-            __syncthreads();
-            for (int wv = 0; wv < (NT + 63) / 64; ++wv) {
-                A0 += red4[wv][0];
-                A1 += red4[wv][1];
-                B0 += red4[wv][2];
-                B1 += red4[wv][3];
-            }
-        }
-        auto none = [](int) { return make_float2(0.f, 0.f); };
-        auto crop = [&](int i, float2 v) {
-            if (a.mode == 4) {
-                if (i >= a.n) return;
-                float y0 = v.x, y1 = v.y;
-                if (i == 0) { y0 += A0; y1 += A1; }
-                if (i == a.n - 1) { y0 += B0; y1 += B1; }
-                o0[i] = y0;
-                if (has1) o1[i] = y1;
-                return;
-            }
-            if (a.mode == 3) {
-                if (i >= a.n) return;
-                const float rf = a.resp_first[i], rl = a.resp_last[i];
-                o0[i] = (v.x + f0 * rf) + l0 * rl;
-                if (has1) o1[i] = (v.y + f1 * rf) + l1 * rl;
-                return;
-            }
-            const int d = i - a.insert;
-            if (d < 0 || d >= a.n) return;
-            if (a.mode == 0) {
-                o0[d] = v.x * a.post0;
-                if (has1) o1[d] = v.y * a.post0;
-            } else {
-                o0[d] = ((v.x * a.post0) * a.post1) * a.post2;
-                if (has1) o1[d] = ((v.y * a.post0) * a.post1) * a.post2;
+                red[t >> 6][0] = sa0;
+                red[t >> 6][1] = sa1;
+                red[t >> 6][2] = sb0;
+                red[t >> 6][3] = sb1;
             }
         };
-        fft_lds2_io<P, NT, true, false, true, false>(line, twl, none, crop);
+        // red is read behind the exchanges of the first and the last stage,
+        // which order the whole block when it has more than one wave
+        auto store = [&](int i, float2 v) {
+            if (i >= a.n) return;
+            float y0 = v.x, y1 = v.y;
+            if (i == 0 || i == a.n - 1) {
+                float A0 = 0.f, A1 = 0.f, B0 = 0.f, B1 = 0.f;
+                for (int wv = 0; wv < (NT + 63) / 64; ++wv) {
+                    A0 += red[wv][0];
+                    A1 += red[wv][1];
+                    B0 += red[wv][2];
+                    B1 += red[wv][3];
+                }
+                if (i == 0) { y0 += A0; y1 += A1; }
+                if (i == a.n - 1) { y0 += B0; y1 += B1; }
+            }
+            o0[i] = y0;
+            if (has1) o1[i] = y1;
+        };
+        fft_filter<P, NT, true>(line, a.tw, a.hs, each(load), reduce, nothing2, to_each(store));
         return;
-    }
-    if (a.mode == 0) {
-        const float f0 = row0[0], l0 = row0[a.n - 1];
-        const float f1 = row1[0], l1 = row1[a.n - 1];
-        for (int i = t; i < P; i += NT) {
-            const float x0 = pb_pad(row0, a.n, i, a.insert, P, a.taper, f0, l0);
-            const float x1 = has1 ? pb_pad(row1, a.n, i, a.insert, P, a.taper, f1, l1) : 0.0f;
-            line[lpad(i)] = make_float2(x0, x1);
-        }
+    } else if (a.mode == 0) {
+        const float f0 = row0[0], l0 = row0[a.n - 1], f1 = row1[0], l1 = row1[a.n - 1];
+        auto load = [&](int i) {
+            return make_float2(pb_pad(row0, a.n, i, a.insert, P, a.taper, f0, l0),
+                               has1 ? pb_pad(row1, a.n, i, a.insert, P, a.taper, f1, l1) : 0.0f);
+        };
+        auto store = [&](int i, float2 v) {
+            const int d = i - a.insert;
+            if (d < 0 || d >= a.n) return;
+            o0[d] = v.x * a.post0;
+            if (has1) o1[d] = v.y * a.post0;
+        };
+        fft_filter<P, NT, false>(line, a.tw, a.hs, each(load), nothing, nothing2, to_each(store));
     } else if (a.mode == 1) {
         const float w0 = a.pre_w ? a.pre_w[r0 / a.rows_per_proj] : 1.0f;
         const float w1 = (a.pre_w && has1) ? a.pre_w[(r0 + 1) / a.rows_per_proj] : 1.0f;
         const float v0 = fdk_row_vv2(a, r0), v1 = fdk_row_vv2(a, r0 + 1);
-        for (int i = t; i < P; i += NT) {
-            const float x0 = fdk_pad(row0, a.n, i, a.insert, P, w0, a, v0);
-            const float x1 = has1 ? fdk_pad(row1, a.n, i, a.insert, P, w1, a, v1) : 0.0f;
-            line[lpad(i)] = make_float2(x0, x1);
-        }
+        auto load = [&](int i) {
+            return make_float2(fdk_pad(row0, a.n, i, a.insert, P, w0, a, v0),
+                               has1 ? fdk_pad(row1, a.n, i, a.insert, P, w1, a, v1) : 0.0f);
+        };
+        auto store = [&](int i, float2 v) {
+            const int d = i - a.insert;
+            if (d < 0 || d >= a.n) return;
+            o0[d] = ((v.x * a.post0) * a.post1) * a.post2;
+            if (has1) o1[d] = ((v.y * a.post0) * a.post1) * a.post2;
+        };
+        fft_filter<P, NT, false>(line, a.tw, a.hs, each(load), nothing, nothing2, to_each(store));
     } else {
         // mode 2, adjoint of mode 0: the scaled rows embedded at nInsert, zeros elsewhere
-        for (int i = t; i < P; i += NT) {
+        auto load = [&](int i) {
             const int d = i - a.insert;
             const bool in = d >= 0 && d < a.n;
-            const float x0 = in ? row0[d] * a.post0 : 0.0f;
-            const float x1 = (in && has1) ? row1[d] * a.post0 : 0.0f;
-            line[lpad(i)] = make_float2(x0, x1);
-        }
-    }
-    __syncthreads();
-    fft_lds2<P, NT, false>(line, twl);
-    for (int i = t; i < P; i += NT) {
-        const float h = a.hs[i];
-        const float2 v = line[lpad(i)];
-        line[lpad(i)] = make_float2(v.x * h, v.y * h);
-    }
-    __syncthreads();
-    fft_lds2<P, NT, true>(line, twl);
-    if (a.mode == 0) {
-        for (int i = t; i < a.n; i += NT) {
-            const float2 v = line[lpad(i + a.insert)];
-            o0[i] = v.x * a.post0;
-            if (has1) o1[i] = v.y * a.post0;
-        }
-    } else if (a.mode == 2) {
+            return make_float2(in ? row0[d] * a.post0 : 0.0f, (in && has1) ? row1[d] * a.post0 : 0.0f);
+        };
+        auto store = [&](int i, float2 v) { line[fft_swz(i)] = v; };   // in place
+        fft_filter<P, NT, false>(line, a.tw, a.hs, each(load), nothing, nothing2, to_each(store));
+        __syncthreads();
         // adjoint of Pad: the tapers fold back onto the first and last sample
         // (left taper at 0..nInsert-1, right taper at P+15-j, inside the
         // FFT window only for j >= 16)
@@ -243,12 +285,12 @@ __global__ __launch_bounds__(NT) void row_filter_kernel2(RowFilterArgs a)
         float sl0 = 0.0f, sl1 = 0.0f, sr0 = 0.0f, sr1 = 0.0f;
         for (int j = t; j < a.insert; j += NT) {
             const float w = a.taper[j];
-            const float2 l = line[lpad(j)];
+            const float2 l = line[fft_swz(j)];
             sl0 += w * l.x;
             sl1 += w * l.y;
             const int jj = P + 15 - j;
             if (jj < P) {
-                const float2 r = line[lpad(jj)];
+                const float2 r = line[fft_swz(jj)];
                 sr0 += w * r.x;
                 sr1 += w * r.y;
             }
@@ -274,18 +316,12 @@ __global__ __launch_bounds__(NT) void row_filter_kernel2(RowFilterArgs a)
             R1 += red[wv][3];
         }
         for (int i = t; i < a.n; i += NT) {
-            const float2 v = line[lpad(i + a.insert)];
+            const float2 v = line[fft_swz(i + a.insert)];
             float y0 = v.x, y1 = v.y;
             if (i == 0) { y0 += L0; y1 += L1; }
             if (i == a.n - 1) { y0 += R0; y1 += R1; }
             o0[i] = y0;
             if (has1) o1[i] = y1;
-        }
-    } else {
-        for (int i = t; i < a.n; i += NT) {
-            const float2 v = line[lpad(i + a.insert)];
-            o0[i] = ((v.x * a.post0) * a.post1) * a.post2;
-            if (has1) o1[i] = ((v.y * a.post0) * a.post1) * a.post2;
         }
     }
 }
@@ -307,15 +343,8 @@ __global__ void fdk_margin_rows_kernel(float *img, int n, int h, long n_proj)
 template <int P>
 static int launch_row_filter(const RowFilterArgs &a, hipStream_t s)
 {
-    // one radix-8 butterfly per thread and pass: P / 8 threads (at most
-    // 1024); measured for the 384 000 rows of 2048 at P = 8192: 6.75 ms with
-    // the padding, spectrum and crop fused into the first and last passes,
-    // 7.8-8.1 ms without, 9.3-9.8 ms with P / 16 threads, 19.75 ms with a
-    // radix-4 FFT; the line split into 4 or 8 wave-local FFTs of length P / 4
-    // or P / 8 (two block barriers per row pair instead of two per pass)
-    // took 11.0 / 8.4 ms (2 / 4 waves per SIMD); radix-16 passes with P / 16
-    // threads 6.52 against 6.49 ms
-    constexpr int NT2 = (P / 8) < 64 ? 64 : ((P / 8) > 1024 ? 1024 : (P / 8));
+    // butterflies of a stage, at least a wave
+    constexpr int NB = (P / 8) < 64 ? 64 : ((P / 8) > 1024 ? 1024 : (P / 8)), NT = filter_threads(P, NB);
     const long pairs = (a.n_rows + 1) / 2;
     if (pairs == 0) return MR_OK;
     if (pairs > 0x7fffffffL) {
@@ -326,11 +355,13 @@ static int launch_row_filter(const RowFilterArgs &a, hipStream_t s)
                                                 : (a.mode == 1 ? "row_filter_fdk" : "row_filter_adjoint"),
                    s);
     MR_REQUIRE((a.mode != 3 && a.mode != 4) || (a.resp_first && a.resp_last), "short filter without responses");
-    const size_t lds = sizeof(float2) * (lds_len(P) + P / 8);
-    if (lds > 65536)
-        MR_HIP(hipFuncSetAttribute((const void *)row_filter_kernel2<P, NT2>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((row_filter_kernel2<P, NT2>), dim3((unsigned)pairs), dim3(NT2), lds, s, a);
+    constexpr size_t lds = sizeof(float2) * P;
+    const bool shortf = a.mode == 3 || a.mode == 4;
+    if (shortf) MR_REQUIRE(2 * (size_t)a.n <= P, "short filter longer than half its line");
+    const void *k = shortf ? (const void *)row_filter_kernel2<P, NB, true> : (const void *)row_filter_kernel2<P, NB, false>;
+    if (lds > 65536) MR_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (shortf) hipLaunchKernelGGL((row_filter_kernel2<P, NB, true>), dim3((unsigned)pairs), dim3(NT), lds, s, a);
+    else hipLaunchKernelGGL((row_filter_kernel2<P, NB, false>), dim3((unsigned)pairs), dim3(NT), lds, s, a);
     MR_HIP(hipGetLastError());
     return MR_OK;
 }
@@ -363,17 +394,33 @@ int run_fdk_margin_rows(float *img, int n, int h, long n_proj, hipStream_t s)
     return MR_OK;
 }
 
-// P twiddles exp(-2 pi i k / P) in double, rounded to float.
+// The radix-8 stages' twiddles exp(-2 pi i m k / span), k < span / 8, for m = 1,
+// 2, 4 and spans P, P/8, ..., in double, rounded to float (P entries, the rest
+// zero).
 std::vector<float> make_twiddles(size_t P)
 {
-    std::vector<float> tw(2 * P);
+    std::vector<float> tw(2 * P, 0.0f);
     const double pi = 3.1415926535897932384626433832795;
-    for (size_t k = 0; k < P; ++k) {
-        const double ang = -2.0 * pi * (double)k / (double)P;
-        tw[2 * k] = (float)std::cos(ang);
-        tw[2 * k + 1] = (float)std::sin(ang);
+    for (int s = 0; s < fft_stages((int)P); ++s) {
+        const size_t span = P >> (3 * s), at = (size_t)fft_tw_offset((int)P, s);
+        for (size_t e = 0; e < 3 * span / 8; ++e) {
+            const size_t m = e / (span / 8), k = e % (span / 8);
+            const double ang = -2.0 * pi * (double)(k << m) / (double)span;
+            tw[2 * (at + e)] = (float)std::cos(ang);
+            tw[2 * (at + e) + 1] = (float)std::sin(ang);
+        }
     }
     return tw;
+}
+
+// A spectrum of P values in the order in which the middle stage's threads
+// read it: point 8 j + m of the digit-reversed line at m P/8 + j.
+std::vector<float> spectrum_order(const std::vector<float> &h)
+{
+    const int P = (int)h.size();
+    std::vector<float> o(h.size());
+    for (int p = 0; p < P; ++p) o[(size_t)(p % 8) * (P / 8) + p / 8] = h[fft_frequency(P, p)];
+    return o;
 }
 
 }  // namespace mr
@@ -530,7 +577,9 @@ extern "C" int mr_filter_plan_create(mr_filter_plan **plan, size_t width, int fi
     hipError_t e = hipMalloc(&p->d_hs, sizeof(float) * P);
     if (e == hipSuccess) e = hipMalloc(&p->d_taper, sizeof(float) * taper.size());
     if (e == hipSuccess) e = hipMalloc(&p->d_tw, sizeof(float2) * P);
-    if (e == hipSuccess) e = hipMemcpy(p->d_hs, hs.data(), sizeof(float) * P, hipMemcpyHostToDevice);
+    // (P may exceed the kernels' lengths when the short form serves)
+    const std::vector<float> hso = mr::spectrum_order(hs);
+    if (e == hipSuccess) e = hipMemcpy(p->d_hs, hso.data(), sizeof(float) * P, hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = hipMemcpy(p->d_taper, taper.data(), sizeof(float) * taper.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->d_tw, tw.data(), sizeof(float) * 2 * P, hipMemcpyHostToDevice);
@@ -540,12 +589,12 @@ extern "C" int mr_filter_plan_create(mr_filter_plan **plan, size_t width, int fi
                          ? mr::short_filter(P, width, n_insert, hs, taper, p->scale, hq, resp, resp_adj)
                          : 0;
     if (Q > 0) {
-        const std::vector<float> twq = mr::make_twiddles(Q);
+        const std::vector<float> twq = mr::make_twiddles(Q), hqo = mr::spectrum_order(hq);
         resp.insert(resp.end(), resp_adj.begin(), resp_adj.end());
         e = hipMalloc(&p->d_hq, sizeof(float) * Q);
         if (e == hipSuccess) e = hipMalloc(&p->d_twq, sizeof(float2) * Q);
         if (e == hipSuccess) e = hipMalloc(&p->d_resp, sizeof(float) * 4 * width);
-        if (e == hipSuccess) e = hipMemcpy(p->d_hq, hq.data(), sizeof(float) * Q, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(p->d_hq, hqo.data(), sizeof(float) * Q, hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(p->d_twq, twq.data(), sizeof(float) * 2 * Q, hipMemcpyHostToDevice);
         if (e == hipSuccess)
             e = hipMemcpy(p->d_resp, resp.data(), sizeof(float) * 4 * width, hipMemcpyHostToDevice);
