@@ -1135,6 +1135,37 @@ static void lds_shape(int nu, int nv, int &zt, int &kc, int &pipe)
     pipe = zt == 8 ? 0 : 1;
 }
 
+// The same for nk projections.  A block's chunks follow one another (barrier,
+// table entries, loads, barrier, sums), and one or two waves per SIMD neither
+// cover those latencies nor issue at full rate (one: 8 cycles per instruction,
+// four: 2.4), so a grid of few blocks takes thinner slice tiles: 4 slices with
+// chunks of 32 while that makes at most 5 blocks per CU, else 8 slices with
+// chunks of 8 where the shape above has fewer than 4 blocks per CU or fewer
+// than 16 slices.  The positions and weights, computed once per tile, are then
+// computed more often.  Exact, in microseconds (shape above, 4, 8 slices):
+// 256^2 x 16 x 180: 71, 48, 55; 128^2 x 16 x 180: 87, 41, 53; 256^2 x 8 x 180:
+// 57, 41, 53; 300^2 x 10 x 700: 207, 166, 196; 256^2 x 24 x 360 (1536 blocks of
+// 4 slices): 145, 150, 108; 400^2 x 16 x 360: 153, 161, 129; 512^2 x 8 x 360:
+// 136, 150, 112; 512^2 x 16 x 360 (1024 blocks): 184, 243, 206.  Below 8 slices
+// the unrolled chunks would add zeros (1024^2 x 4 x 400: 302 above, 363 with 8).
+// Fewer than 64 projections are a few chunks whichever way and keep the shape
+// above.
+static void lds_shape_nk(int nu, int nv, int nk, int &zt, int &kc, int &pipe)
+{
+    lds_shape(nu, nv, zt, kc, pipe);
+    const long tiles = (long)((nu + 15) / 16) * ((nu + 15) / 16);
+    if (nk < 64 || zt == 32) return;
+    if (tiles * ((nv + 3) / 4) <= 1280) {
+        zt = 4;
+        kc = 32;
+        pipe = 0;
+    } else if (nv >= 8 && (zt == 8 || tiles * ((nv + 15) / 16) < 1024)) {
+        zt = 8;
+        kc = 8;
+        pipe = 1;
+    }
+}
+
 // impl 0: direct global gathers (MultiProjBP's second column read at its own
 // offset, which differs from the staged layout when slices % 4 != 0);
 // impl 1: LDS-staged tiles.  exact: the reference's float operation order
@@ -1172,15 +1203,17 @@ int run_bp(const BpArgs &a, int interp, int impl, int exact, hipStream_t s)
         return interp == 0 ? launch_bp<4, 0>(a, s) : launch_bp<4, 1>(a, s);
     }
     int zt, kc, pipe;
-    lds_shape(a.nu, a.nv, zt, kc, pipe);
+    lds_shape_nk(a.nu, a.nv, a.nk, zt, kc, pipe);
     if (zt == 32) return launch_bp_lds_mode<32, 4, 1>(a, interp, exact, s);
     if (zt == 16) return launch_bp_lds_mode<16, 8, 1>(a, interp, exact, s);
+    if (zt == 4) return launch_bp_lds_mode<4, 32, 0>(a, interp, exact, s);
+    if (pipe) return launch_bp_lds_mode<8, 8, 1>(a, interp, exact, s);
     return launch_bp_lds_mode<8, 16, 0>(a, interp, exact, s);
 }
 
 // The kernel run_bp launches for these settings, e.g.
-// "bp_lds_kernel<32,0,false,4,1> order=1 sw=4".
-std::string describe_bp(int nu, int nv, int interp, int impl, int exact, int tilt)
+// "bp_lds_kernel<32,0,false,4,1> order=1 sw=4" (nk 0: for few projections).
+std::string describe_bp(int nu, int nv, int nk, int interp, int impl, int exact, int tilt)
 {
     if (tilt != 0 && impl == 1) {
         int zt, kc, pipe;
@@ -1198,7 +1231,7 @@ std::string describe_bp(int nu, int nv, int interp, int impl, int exact, int til
         return "bp_kernel<" + std::to_string(zt) + "," + std::to_string(interp) + ">";
     }
     int zt, kc, pipe;
-    lds_shape(nu, nv, zt, kc, pipe);
+    lds_shape_nk(nu, nv, nk, zt, kc, pipe);
     const long n = (long)((nu + 15) / 16) * ((nu + 15) / 16) * ((nv + zt - 1) / zt);
     return "bp_lds_kernel<" + std::to_string(zt) + "," + std::to_string(interp) + "," +
            ((interp == 1 || exact) ? "true" : "false") + "," + std::to_string(kc) + "," + std::to_string(pipe) +
@@ -1407,7 +1440,8 @@ extern "C" int mr_bp_plan_kernel(const mr_bp_plan *plan, char *name, size_t len)
     // with tables loaded, the form their projection count selects
     const std::string d = plan->loaded && mr::plan_bpm(plan, plan->loaded_nk, tile)
                               ? "bp_mfma_kernel tile=" + std::to_string(tile)
-                              : mr::describe_bp((int)plan->p.width, (int)plan->p.slices, plan->p.interp, plan->impl,
+                              : mr::describe_bp((int)plan->p.width, (int)plan->p.slices,
+                                                plan->loaded ? (int)plan->loaded_nk : 0, plan->p.interp, plan->impl,
                                                 plan->p.fused ? 0 : 1, plan->tilt);
     std::snprintf(name, len, "%s", d.c_str());
     return MR_OK;
