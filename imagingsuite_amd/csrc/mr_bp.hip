@@ -1155,7 +1155,7 @@ static void lds_shape_nk(int nu, int nv, int nk, int &zt, int &kc, int &pipe)
     lds_shape(nu, nv, zt, kc, pipe);
     const long tiles = (long)((nu + 15) / 16) * ((nu + 15) / 16);
     if (nk < 64 || zt == 32) return;
-    if (tiles * ((nv + 3) / 4) <= 1280) {
+    if (tiles * ((nv + 3) / 4) <= 1280 && (nv >= 8 || tiles <= 512)) {
         zt = 4;
         kc = 32;
         pipe = 0;
