@@ -758,7 +758,7 @@ def joseph_leg(steps, full, fp64_gd=False):
 
     out = {"workload": "matched Joseph pair and FBP pair, 1024^2 x 64 slices x 900 angles",
            "A": {"ms": round(ms_a, 3), "GUPS": round(upd / (ms_a / 1e3) / 1e9, 2),
-                 "roofline": rl("joseph_forward_lds2_kernel<32>", ka["joseph_forward"][0])},
+                 "roofline": rl("joseph_forward_dma_kernel<32,1>", ka["joseph_forward"][0])},
            "AT": {"ms": round(ms_t, 3), "GUPS": round(upd / (ms_t / 1e3) / 1e9, 2),
                   "roofline": rl("joseph_adjoint_lds_kernel<32,4>", kt["joseph_adjoint"][0])}}
     # gradient through filtered back-projection: F^T BP^T

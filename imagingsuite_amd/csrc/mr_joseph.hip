@@ -255,26 +255,37 @@ __global__ __launch_bounds__(256) void joseph_forward_lds_kernel(JosephArgs a, c
             make_float4(acc[4 * g] * inv_m, acc[4 * g + 1] * inv_m, acc[4 * g + 2] * inv_m, acc[4 * g + 3] * inv_m);
 }
 
-// The same forward with one barrier per line.  The block first computes,
+// The same forward with one barrier per R lines.  The block first computes,
 // for every line, the span of its rays' crossings (the minimum and maximum
-// floor(crossing) over the edge rays, the first and last valid bin of each
-// of its angles, with the same float expression) into LDS; the per-line
-// loop then stages line L + 1 into one buffer while its rays interpolate
-// line L from the other, and a single barrier separates the lines.  Staged
-// values, offsets and the order of the sums are those of
-// joseph_forward_lds_kernel, so the projections are bit-identical to it.
-// Dynamic LDS: 2 N ints (the spans).  Bounded to five waves per SIMD, which
-// the LDS allows (1024^2 x 64 x 900: 6.8 ms, 7.7 ms at the four the
-// registers would otherwise give).
-template <int ZT>
-__global__ __launch_bounds__(256, 5) void joseph_forward_lds2_kernel(JosephArgs a, const int4 *__restrict__ chunks,
-                                                                  const int *__restrict__ order, int n_chunks,
-                                                                  int nbt, int nzs)
+// floor(crossing) over the edge rays, the first and last valid bin of each of
+// its angles, with the same float expression) into LDS; while its rays
+// interpolate R lines from one buffer, direct loads stage the next R into the
+// other.  A line is staged by 256 / R threads in 16-byte chunks, G of a
+// position's slices and one unused (an offset past the range loads zeros
+// there), so that positions lie ZT + 4 floats apart; the spans are read two
+// steps ahead.  Slice counts are any multiple of 4: groups beyond the last are
+// staged as zeros and not stored.  Values and order of the sums are those of
+// joseph_forward_lds_kernel, or with direct set of joseph_forward_kernel, which
+// adds the column class's terms in another order: bit-identical to either.
+//
+// What limits it is the latency of a line (position, LDS address, LDS read,
+// barrier) at 3 to 5 waves per SIMD; the form before staged through registers
+// and read its spans when it needed them.  Projection in microseconds, before
+// and now: 512^2 x 16 x 360 (R = 2) 430, 260; 512^2 x 32 x 360 (R = 1) 567, 378
+// (502 with R = 2); 1024^2 x 64 x 200 5302, 3847 (4976 with R = 2); slice counts
+// that took joseph_forward_kernel: 300^2 x 20 x 200 461, 136; 700^2 x 8 x 200
+// (8 slices, R = 4) 924, 333.
+// Dynamic LDS: N + 3 R spans.
+template <int ZT, int R>
+__global__ __launch_bounds__(256, R == 4 ? 4 : 5) void joseph_forward_dma_kernel(
+    JosephArgs a, const int4 *__restrict__ chunks, const int *__restrict__ order, int n_chunks, int nbt, int nzs,
+    int direct)
 {
-    constexpr int NB = kFwdNB, KA = kFwdKA, W = kFwdW, RS = ZT + 4, G = ZT / 4;
-    __shared__ float seg[2][W][RS];
-    __shared__ float4 ep[2 * KA];   // edge rays: (a0, b1, cn, inv)
-    extern __shared__ int spans[];  // lo of line L at [L], hi at [N + L]
+    constexpr int NB = kFwdNB, KA = kFwdKA, W = kFwdW, G = ZT / 4, GP = G + 1, RS = 4 * GP;
+    constexpr int TL = 256 / R, NE = (W * GP + TL - 1) / TL;
+    __shared__ __align__(16) float seg[2][R][W * RS];
+    __shared__ float4 ep[2 * KA];    // edge rays: (a0, b1, cn, inv)
+    extern __shared__ int2 jspans[]; // [lo, hi] of line L; lines N .. N + 3 R - 1 are dead
     const int total = n_chunks * nbt * nzs;
     const int per = (total + 7) >> 3;
     const int b = (int)blockIdx.x;
@@ -299,9 +310,11 @@ __global__ __launch_bounds__(256, 5) void joseph_forward_lds2_kernel(JosephArgs 
     const int z0 = zs * ZT;
     const bool rows = ch.z == 0;
     // crossing of line L: ((a0 + b1 (L+1)) + cn) * inv - 1
-    const float a0 = rows ? su : -su, b1 = rows ? c : s;
+    const bool own = direct && !rows;
+    const float b1 = rows ? c : s;
     const float fn = (float)n;
-    const float cn = rows ? -fn : fn;
+    const float a0 = own ? fn - su : (rows ? su : -su);
+    const float cn = own ? 0.0f : (rows ? -fn : fn);
     const float inv = rows ? 1.0f / s : 1.0f / c;
     const size_t strideL = rows ? (size_t)N * a.nz : (size_t)a.nz;
     const size_t strideP = rows ? (size_t)a.nz : (size_t)N * a.nz;
@@ -311,77 +324,85 @@ __global__ __launch_bounds__(256, 5) void joseph_forward_lds2_kernel(JosephArgs 
         const int en = min(bt * NB + ((tid & 1) ? NB - 1 : 0), a.nd - 1);
         const float4 et = a.tab[order[ch.x + min(ea, ch.y - 1)]];
         const float efn = (float)en;
-        ep[tid] = make_float4(rows ? et.x : -et.x, rows ? et.y : et.z, rows ? -efn : efn,
-                              rows ? 1.0f / et.z : 1.0f / et.y);
+        ep[tid] = make_float4(own ? efn - et.x : (rows ? et.x : -et.x), rows ? et.y : et.z,
+                              own ? 0.0f : (rows ? -efn : efn), rows ? 1.0f / et.z : 1.0f / et.y);
     }
     __syncthreads();
     const int ne = 2 * ch.y;
-    for (int L = tid; L < N; L += 256) {
+    for (int L = tid; L < N + 3 * R; L += 256) {
         int lo = 0x7fffffff, hi = -0x7fffffff;
-        for (int e = 0; e < ne; ++e) {
+        for (int e = 0; L < N && e < ne; ++e) {
             const float4 q = ep[e];
             const int p0 = (int)floorf(((q.x + q.y * (float)(L + 1)) + q.z) * q.w - 1.0f);
             lo = min(lo, p0);
             hi = max(hi, p0);
         }
-        spans[L] = lo;
-        spans[N + L] = hi;
+        // a line is dead when no ray of the block crosses the volume on it
+        jspans[L] = hi >= -1 && lo < N ? make_int2(lo, hi) : make_int2(0x7fffffff, 0x7fffffff);
     }
     __syncthreads();
     float acc[ZT];
 #pragma unroll
     for (int z = 0; z < ZT; ++z) acc[z] = 0.0f;
-    // a line is skipped when no ray of the block crosses the volume on it
-    auto live = [&](int L) { return spans[N + L] >= -1 && spans[L] < N; };
-    // only the voxels a line's rays read: lo .. hi + 1.  fetch() issues the
-    // global loads of line L into registers, put() writes them to seg[buf]
-    // one line later, so the loads of line L + 2 are in flight while line L
-    // is consumed.  Element e = tid + 256 i is (position lo + e / G, slice
-    // group e % G).
-    constexpr int NE = (W * G + 255) / 256;
-    float4 pre[NE];
-    auto fetch = [&](int L) {
-        const int lo = spans[L], nj = min(spans[N + L] - lo + 2, W);
-        const float *line = a.src + (size_t)L * strideL + z0;
+    // chunks of this thread: position j and byte offset from the line's first position
+    const int sr = __builtin_amdgcn_readfirstlane(tid / TL), le = tid - sr * TL;
+    int st_j[NE];
+    unsigned st_off[NE];
 #pragma unroll
-        for (int i = 0; i < NE; ++i) {
-            const int e = tid + 256 * i;
-            const int j = e / G, g = e - j * G;
-            const int p = lo + j;
-            pre[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (e < nj * G && p >= 0 && p < N)
-                pre[i] = *reinterpret_cast<const float4 *>(line + (size_t)p * strideP + 4 * g);
-        }
-    };
-    auto put = [&](int L, int buf) {
-        const int nj = min(spans[N + L] - spans[L] + 2, W);
-#pragma unroll
-        for (int i = 0; i < NE; ++i) {
-            const int e = tid + 256 * i;
-            const int j = e / G, g = e - j * G;
-            if (e < nj * G) *reinterpret_cast<float4 *>(&seg[buf][j][4 * g]) = pre[i];
-        }
-    };
-    if (live(0)) {
-        fetch(0);
-        put(0, 0);
+    for (int i = 0; i < NE; ++i) {
+        const int e = le + TL * i, j = e / GP, g = e - j * GP;
+        const bool used = e < W * GP && g < G && z0 + 4 * g < a.nz;
+        st_j[i] = j;
+        st_off[i] = used ? (unsigned)j * (unsigned)(4 * strideP) + 16u * (unsigned)g : 0x80000000u;
     }
-    if (N > 1 && live(1)) fetch(1);
+    auto stage = [&](int L, int2 sp, float *dst) {
+        if (sp.x == 0x7fffffff) return;
+        const int nj = min(sp.y - sp.x + 2, W);   // only the voxels a line's rays read: lo .. hi + 1
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(a.src + ((long)L * (long)strideL + (long)sp.x * (long)strideP + z0)), (short)0, 0x7FFFFFFF,
+            0x00020000);
+        const int w64 = __builtin_amdgcn_readfirstlane(le & ~63);
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            if (w64 + TL * i >= nj * GP) break;
+            const unsigned off = (unsigned)(sp.x + st_j[i]) < (unsigned)N ? st_off[i] : 0x80000000u;
+            if (le + TL * i < W * GP)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rs, (__attribute__((address_space(3))) void *)(dst + 4 * (w64 + TL * i)), 16, off, 0, 0, 0);
+        }
+    };
+    auto span = [&](int L) {
+        const int2 v = jspans[L];
+        return make_int2(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y));
+    };
+    int2 cur[R], nxt[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        cur[r] = span(r);
+        nxt[r] = span(R + r);
+    }
+    stage(sr, span(sr), seg[0][sr]);
     __syncthreads();
-    for (int L = 0; L < N; ++L) {
-        const int buf = L & 1;
-        // line L + 1: loaded during the previous line, into the other buffer
-        if (L + 1 < N && live(L + 1)) put(L + 1, buf ^ 1);
-        if (L + 2 < N && live(L + 2)) fetch(L + 2);
-        if (live(L)) {
-            const float pf = ((a0 + b1 * (float)(L + 1)) + cn) * inv - 1.0f;
+    for (int L0 = 0, buf = 0; L0 < N; L0 += R, buf ^= 1) {
+        int2 far[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) far[r] = jspans[L0 + 2 * R + r];
+        int2 mine = nxt[0];
+#pragma unroll
+        for (int r = 1; r < R; ++r)
+            if (sr == r) mine = nxt[r];
+        stage(L0 + R + sr, mine, seg[buf ^ 1][sr]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (cur[r].x == 0x7fffffff) continue;
+            const float pf = ((a0 + b1 * (float)(L0 + r + 1)) + cn) * inv - 1.0f;
             const float fl = floorf(pf);
             const int p0 = (int)fl;
             const float f = pf - fl;
             const float w0 = (p0 >= 0 && p0 < N) ? 1.0f - f : 0.0f;
             const float w1 = (p0 + 1 >= 0 && p0 + 1 < N) ? f : 0.0f;
-            const int j = min(max(p0 - spans[L], 0), W - 2);
-            const float *v0 = &seg[buf][j][0];
+            const int j = min(max(p0 - cur[r].x, 0), W - 2);
+            const float *v0 = &seg[buf][r][j * RS];
             const float *v1 = v0 + RS;
 #pragma unroll
             for (int g = 0; g < G; ++g) {
@@ -393,14 +414,20 @@ __global__ __launch_bounds__(256, 5) void joseph_forward_lds2_kernel(JosephArgs 
                 acc[4 * g + 3] = __builtin_fmaf(w1, x1.w, __builtin_fmaf(w0, x0.w, acc[4 * g + 3]));
             }
         }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            cur[r] = nxt[r];
+            nxt[r] = make_int2(__builtin_amdgcn_readfirstlane(far[r].x), __builtin_amdgcn_readfirstlane(far[r].y));
+        }
         __syncthreads();
     }
     if (!active) return;
     float *out = a.dst + ((size_t)ang * a.nd + n) * a.nz + z0;
 #pragma unroll
     for (int g = 0; g < G; ++g)
-        *reinterpret_cast<float4 *>(out + 4 * g) =
-            make_float4(acc[4 * g] * inv_m, acc[4 * g + 1] * inv_m, acc[4 * g + 2] * inv_m, acc[4 * g + 3] * inv_m);
+        if (z0 + 4 * g < a.nz)
+            *reinterpret_cast<float4 *>(out + 4 * g) = make_float4(acc[4 * g] * inv_m, acc[4 * g + 1] * inv_m,
+                                                                   acc[4 * g + 2] * inv_m, acc[4 * g + 3] * inv_m);
 }
 
 // Adjoint: one thread per (x, y) voxel column and ZT slices.
@@ -495,7 +522,7 @@ __global__ __launch_bounds__(256) void joseph_adjoint_lds_kernel(JosephArgs a, i
             const int bb = rr / G, g = rr - bb * G;
             const int col = sb0[kk] + bb;
             float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (col >= 0 && col < a.nd)
+            if (col >= 0 && col < a.nd && z0 + 4 * g < a.nz)
                 v = *reinterpret_cast<const float4 *>(a.src + ((size_t)(kb + kk) * a.nd + col) * a.nz + z0 + 4 * g);
             *reinterpret_cast<float4 *>(&sm[kk][bb][4 * g]) = v;
         }
@@ -530,8 +557,9 @@ __global__ __launch_bounds__(256) void joseph_adjoint_lds_kernel(JosephArgs a, i
     float *out = a.dst + ((size_t)y * N + x) * a.nz + z0;
 #pragma unroll
     for (int g = 0; g < G; ++g)
-        *reinterpret_cast<float4 *>(out + 4 * g) =
-            make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
+        if (z0 + 4 * g < a.nz)
+            *reinterpret_cast<float4 *>(out + 4 * g) =
+                make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
 }
 
 std::vector<float> joseph_tables(const mr_joseph_geom &g, const float *angles, size_t n_ang)
@@ -670,55 +698,68 @@ int joseph_launch(const mr_joseph_geom *g, const float *src, float *dst, const J
 {
     mr::JosephArgs a{src, dst, dt.tab, (int)g->nx, (int)g->nz, (int)g->n_det, (int)n_ang};
     constexpr int ZT = 4;
-    // ZT = 16 when the slice count allows it
     if (forward) {
         mr::ProfScope prof("joseph_forward", s);
-        if (g->nz % 16 == 0 && dt.n_chunks > 0) {
-            // 32 slices per block when the slice count allows (measured at
-            // 1024^2 x 64 x 900: 7.7 ms against 8.4 with 16)
-            const int zt = g->nz % 32 == 0 ? 32 : 16;
-            const int nbt = (int)((g->n_det + kFwdNB - 1) / kFwdNB), nzs = (int)(g->nz / zt);
-            const long total = (long)dt.n_chunks * nbt * nzs;
+        // The staged form with direct loads: 32 slices and a line per barrier
+        // where the slice count is a multiple of 32, 8 slices and 4 lines up to
+        // 8 slices, else 16 slices and 2 lines; while its spans fit in LDS
+        // beside the lines (64 KB) and a staged line's offsets in 32 bits.
+        const int zt = g->nz % 32 == 0 ? 32 : (g->nz > 8 ? 16 : 8), R = zt == 32 ? 1 : (zt == 16 ? 2 : 4);
+        const int nbt = (int)((g->n_det + kFwdNB - 1) / kFwdNB), nzs = (int)((g->nz + zt - 1) / zt);
+        const long total = (long)dt.n_chunks * nbt * nzs;
+        const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
+        const size_t dyn = sizeof(int2) * (g->nx + 3 * R);
+        const size_t fixed = sizeof(float) * 2 * R * kFwdW * (zt + 4) + sizeof(float4) * 2 * kFwdKA;
+        const int direct = g->nz % 16 == 0 ? 0 : 1;
+        // (Slice counts that are not a multiple of 16 from 128 blocks: with fewer,
+        // joseph_forward_kernel's larger grid wins - 100^2 x 28 x 50, 56 blocks:
+        // 20 against 42 us, 200^2 x 4 x 90, 78: 48 against 46.)
+        if (dt.n_chunks > 0 && total < (1L << 31) - 8 && dyn + fixed <= 65536 && g->nx * g->nz < 6500000 &&
+            (!direct || total >= 128)) {
+            if (zt == 32)
+                hipLaunchKernelGGL((mr::joseph_forward_dma_kernel<32, 1>), grid, dim3(256), dyn, s, a, dt.chunks,
+                                   dt.order, dt.n_chunks, nbt, nzs, direct);
+            else if (zt == 16)
+                hipLaunchKernelGGL((mr::joseph_forward_dma_kernel<16, 2>), grid, dim3(256), dyn, s, a, dt.chunks,
+                                   dt.order, dt.n_chunks, nbt, nzs, direct);
+            else
+                hipLaunchKernelGGL((mr::joseph_forward_dma_kernel<8, 4>), grid, dim3(256), dyn, s, a, dt.chunks,
+                                   dt.order, dt.n_chunks, nbt, nzs, direct);
+        } else if (g->nz % 16 == 0 && dt.n_chunks > 0) {
             MR_REQUIRE(total < (1L << 31) - 8, "Joseph forward grid too large");
-            const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
-            if (g->nx <= 4096) {
-                // one barrier per line (spans precomputed in LDS, 8 bytes per line)
-                const size_t dyn = sizeof(int) * 2 * g->nx;
-                if (zt == 32)
-                    hipLaunchKernelGGL((mr::joseph_forward_lds2_kernel<32>), grid, dim3(256), dyn, s, a, dt.chunks,
-                                       dt.order, dt.n_chunks, nbt, nzs);
-                else
-                    hipLaunchKernelGGL((mr::joseph_forward_lds2_kernel<16>), grid, dim3(256), dyn, s, a, dt.chunks,
-                                       dt.order, dt.n_chunks, nbt, nzs);
-            } else if (zt == 32) {
-                // wider volumes: the span table would not fit beside the staging
-                // buffers; the per-line form gives the same bits
+            // larger volumes: the per-line form gives the same bits
+            if (zt == 32)
                 hipLaunchKernelGGL((mr::joseph_forward_lds_kernel<32, kFwdR>), grid, dim3(256), 0, s, a, dt.chunks,
                                    dt.order, dt.n_chunks, nbt, nzs);
-            } else {
+            else
                 hipLaunchKernelGGL((mr::joseph_forward_lds_kernel<16, kFwdR>), grid, dim3(256), 0, s, a, dt.chunks,
                                    dt.order, dt.n_chunks, nbt, nzs);
-            }
         } else {
-            // slice counts that are not a multiple of 16: direct ray-driven gathers
+            // other slice counts, few blocks or a large volume: direct ray-driven gathers
             dim3 grid((unsigned)((g->n_det + 63) / 64), (unsigned)((n_ang + 3) / 4), (unsigned)(g->nz / ZT));
             hipLaunchKernelGGL(mr::joseph_forward_kernel<ZT>, grid, dim3(256), 0, s, a);
         }
     } else {
         mr::ProfScope prof("joseph_adjoint", s);
-        const int ntx = (int)((g->nx + 15) / 16);
-        if (g->nz % 32 == 0) {
-            const long nt = (long)ntx * ntx * (long)(g->nz / 32);
-            hipLaunchKernelGGL((mr::joseph_adjoint_lds_kernel<32, 4>), dim3((unsigned)(8 * ((nt + 7) / 8))), dim3(256),
-                               0, s, a, ntx, ntx, (int)(g->nz / 32));
-        } else if (g->nz % 16 == 0) {
-            const long nt = (long)ntx * ntx * (long)(g->nz / 16);
-            hipLaunchKernelGGL((mr::joseph_adjoint_lds_kernel<16, 8>), dim3((unsigned)(8 * ((nt + 7) / 8))), dim3(256),
-                               0, s, a, ntx, ntx, (int)(g->nz / 16));
+        // slice tiles of 32 where the count is a multiple of it, 8 up to 8
+        // slices, else 16 (a rest is staged as zeros).  Slice counts that are not
+        // a multiple of 16 take the voxel-driven kernel, which gives the same
+        // bits, below 512 tiles: 128^2 x 24 x 60 (128 tiles) 18 against 28 us,
+        // 300^2 x 20 x 200 (722) 125 against 101, 700^2 x 8 x 200 220 against 112.
+        const int zt = g->nz % 32 == 0 ? 32 : (g->nz > 8 ? 16 : 8);
+        const int ntx = (int)((g->nx + 15) / 16), ntz = (int)((g->nz + zt - 1) / zt);
+        const long nt = (long)ntx * ntx * ntz;
+        const dim3 grid((unsigned)(8 * ((nt + 7) / 8)));
+        if (nt >= (1L << 30) || (g->nz % 16 != 0 && nt < 512)) {
+            // (also more tiles than the tile numbers hold)
+            dim3 g3((unsigned)ntx, (unsigned)ntx, (unsigned)(g->nz / ZT));
+            hipLaunchKernelGGL(mr::joseph_adjoint_kernel<ZT>, g3, dim3(256), 0, s, a);
+        } else if (zt == 32) {
+            hipLaunchKernelGGL((mr::joseph_adjoint_lds_kernel<32, 4>), grid, dim3(256), 0, s, a, ntx, ntx, ntz);
+        } else if (zt == 16) {
+            hipLaunchKernelGGL((mr::joseph_adjoint_lds_kernel<16, 8>), grid, dim3(256), 0, s, a, ntx, ntx, ntz);
         } else {
-            // slice counts that are not a multiple of 16: voxel-driven gathers
-            dim3 grid((unsigned)((g->nx + 15) / 16), (unsigned)((g->nx + 15) / 16), (unsigned)(g->nz / ZT));
-            hipLaunchKernelGGL(mr::joseph_adjoint_kernel<ZT>, grid, dim3(256), 0, s, a);
+            hipLaunchKernelGGL((mr::joseph_adjoint_lds_kernel<8, 16>), grid, dim3(256), 0, s, a, ntx, ntx, ntz);
         }
     }
     MR_HIP(hipGetLastError());
