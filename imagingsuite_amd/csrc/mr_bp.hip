@@ -707,10 +707,15 @@ static int launch_bp(const BpArgs &a, hipStream_t s)
 // whose contributing voxels, for every block of kAdjNB detector bins, lie
 // within kAdjW - 6 voxels on every line.  A block takes kAdjNB bins x one
 // chunk of up to kAdjKA projections x ZT slices, one (bin, projection) per
-// thread, and walks the lines (rows or columns) of the volume: each line's
-// span of candidate voxels is staged into LDS (zeros outside the circle
-// mask) while the previous line is consumed, one barrier per line; the
-// global loads of a line are issued two lines ahead, into registers.
+// thread, and walks the lines (rows or columns) of the volume R at a time: each
+// line's span of candidate voxels is staged into LDS by direct loads while the
+// previous R lines are consumed, one barrier per R lines, and the spans are
+// read two steps ahead.  (Staged through registers, a line at a time, spans
+// read when needed and one window position after the other: 1024^2 x 64 x 900
+// 8.4 against 7.1 ms, 512^2 x 16 x 360 0.63 against 0.50, 256^2 x 36 x 180 -
+// then nine 4-slice tiles instead of three of 16 - 0.44 against 0.23.)  Bound
+// by the LDS reads of the windows (about 55 % of the cycles before, 65 % now)
+// and the latency of a line.
 //
 // On one line the detector position u is monotone along the line with slope
 // |sin| (or |cos|) >= 1/sqrt 2, so the voxels a bin receives from form one
@@ -722,14 +727,12 @@ static int launch_bp(const BpArgs &a, hipStream_t s)
 // nearest neighbour), zero for window positions outside the run.  Without
 // the fix-up the linear form can miss a voxel at a run's end whose weight is
 // within the estimate's rounding of 0 (1024^2 x 64 x 900: 0.02 % of the
-// outputs change, by at most 1.2e-7; 9.2 against 9.7 ms).  Bin 1 of the linear form also takes u in
-// (-1, 0), which (int) truncates to bin 0 (a run of up to 5), and bin nu - 1
-// takes only n = nu - 2: bp_adjoint_edge_kernel computes those two bins.  A
-// line whose staged span holds no voxel of the mask is skipped.  The volume is
+// outputs change, by at most 1.2e-7; the fix-up costs 5 %).  Bin 1 of the
+// linear form also takes u in (-1, 0), which (int) truncates to bin 0 (a run of
+// up to 5), and bin nu - 1 takes only n = nu - 2: bp_adjoint_edge_kernel
+// computes those two bins.  A line whose staged span holds no voxel of the mask is skipped.  The volume is
 // read once per chunk; slices at or beyond 4*(nv/4) and dropped projections
-// get no gradient (the caller zero-fills the output first).  1024^2 x 64 x
-// 900 (all projections): 9.6 ms with the hat against 11.5 ms with the
-// forward's operations for every weight.
+// get no gradient (the caller zero-fills the output first).
 constexpr int kAdjNB = 16, kAdjKA = 16, kAdjW = 80;
 
 // The forward's weight of the voxel at position p (1-based) of line L for
@@ -748,7 +751,7 @@ __device__ __forceinline__ float adj_weight(float su, float c, float s, bool row
     return (in && n == u) ? w_n : ((INTERP == 0 && in && n == u - 1) ? wb : 0.0f);
 }
 
-template <int INTERP, int ZT>
+template <int INTERP, int ZT, int R>
 __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict__ g, float *__restrict__ out,
                                                          const float4 *__restrict__ tab,
                                                          const int2 *__restrict__ mask,
@@ -757,13 +760,14 @@ __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict
                                                          const float *__restrict__ wts,
                                                          const int4 *__restrict__ chunks,
                                                          const int *__restrict__ order, int n_chunks, int nbt,
-                                                         int nzs, int nu, int nv)
+                                                         int nzs, int nu, int nv, int nz4)
 {
-    constexpr int NB = kAdjNB, KA = kAdjKA, W = kAdjW, RS = ZT + 4, G = ZT / 4;
-    __shared__ float seg[2][W][RS];
+    constexpr int NB = kAdjNB, KA = kAdjKA, W = kAdjW, G = ZT / 4, GP = G + 1, RS = 4 * GP;
+    constexpr int TL = 256 / R;     // threads that stage a line
+    __shared__ __align__(16) float seg[2][R][W][RS];
     __shared__ float4 ep[2 * KA];   // edge rays: (su, c, s, lower u bound)
     __shared__ float eu[2 * KA];    // edge rays: upper u bound
-    extern __shared__ int2 spans[]; // line L (1-based) at [L - 1]: staged positions [lo, hi], 1-based
+    extern __shared__ int2 spans[]; // line L (1-based) at [L - 1]: staged positions [lo, hi], 1-based; lines nu + 1 .. nu + 3 R: none
     const int total = n_chunks * nbt * nzs;
     const int per = (total + 7) >> 3;
     const int b = (int)blockIdx.x;
@@ -803,7 +807,7 @@ __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict
         ep[tid] = make_float4(et.x, et.y, et.z, eb <= 1 ? -1.0f : efu - 1.0f);
         eu[tid] = efu + 1.0f;
     }
-    for (int e = tid; e < 2 * W * RS; e += 256) (&seg[0][0][0])[e] = 0.0f;
+    if (tid < 3 * R) spans[nu + tid] = make_int2(1, 0);
     __syncthreads();
     // Per line the positions the block's runs can reach (the edge rays'
     // ranges bound every ray's range), cut to the line's run of mask voxels
@@ -837,70 +841,36 @@ __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict
     float acc[ZT];
 #pragma unroll
     for (int z = 0; z < ZT; ++z) acc[z] = 0.0f;
-    auto live = [&](int L) {
-        const int2 sp = spans[L - 1];
-        return sp.x <= sp.y;
-    };
-    // Staging of a line's span in two halves: fetch() issues the global
-    // loads of line L into registers, put() writes them to seg[buf] one
-    // iteration later, so the loads of line L + 2 are in flight while line L
-    // is consumed.  Element e = tid + 256 i is (position j = e / G, slice
-    // group e % G).
-    constexpr int NE = (W * G + 255) / 256;
-    float4 pre[NE];
-    // When the whole volume lies within 2^31 bytes the loads go through a
-    // buffer resource over it with 32-bit byte offsets, whose per-element
-    // part (position j of the span, slice group gq) is computed once here:
-    // a line then costs one add per element instead of 64-bit address
-    // arithmetic.  Elements past the span get an offset past the range
-    // (zeros; put() does not store them).
-    const size_t vol_bytes = (size_t)nu * nu * nv * sizeof(float);
-    const bool off32 = vol_bytes < 0x7FFFFFF0u;
-    const unsigned stepb = rows ? (unsigned)nv * 4u : (unsigned)(off32 ? (size_t)nu * nv * 4 : 0);
-    unsigned st_off[NE];
+    // Staging of a line's span by direct loads into LDS, in 16-byte chunks: G of
+    // a position's slices and one lane without a load, so that positions lie
+    // ZT + 4 floats apart.
+    constexpr int NE = (W * GP + TL - 1) / TL;
+    const int sr = __builtin_amdgcn_readfirstlane(tid / TL), le = tid - sr * TL;
+    int st_j[NE];
+    size_t st_off[NE];
 #pragma unroll
     for (int i = 0; i < NE; ++i) {
-        const int e = tid + 256 * i;
-        const int j = e / G, gq = e - j * G;
-        st_off[i] = (unsigned)j * stepb + 4u * (unsigned)(z0 + 4 * gq);
+        const int j = (le + TL * i) / GP, gq = (le + TL * i) - j * GP;
+        st_j[i] = gq < G && z0 + 4 * gq < nz4 ? j : W;   // slices past the last group: nothing, and not stored
+        st_off[i] = (size_t)j * (rows ? (size_t)nv : (size_t)nu * nv) + z0 + 4 * gq;
     }
-    const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)g, (short)0, off32 ? (int)vol_bytes : 0x7FFFFFF0, 0x00020000);
-    auto fetch = [&](int L) {
-        const int2 sp = spans[L - 1];
-        const int n_el = (min(sp.y - sp.x, W - 1) + 1) * G;
-        if (off32) {
-            // voxel (position p, line L) at ((y - 1) nu + (x - 1)) nv
-            const unsigned lineb = rows ? (unsigned)(L - 1) * (unsigned)nu * stepb : (unsigned)(L - 1) * (unsigned)nv * 4u;
-            const unsigned pb = lineb + (unsigned)(sp.x - 1) * stepb;
-#pragma unroll
-            for (int i = 0; i < NE; ++i) {
-                const int e = tid + 256 * i;
-                const unsigned off = e < n_el ? pb + st_off[i] : 0x80000000u;
-                pre[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(vrs, off, 0, 0));
-            }
-            return;
-        }
-        const size_t base = rows ? (size_t)(L - 1) * nu * nv : (size_t)(L - 1) * nv;
-        const size_t step = rows ? (size_t)nv : (size_t)nu * nv;
+    const int w64 = __builtin_amdgcn_readfirstlane(le & ~63);
+    auto stage = [&](int L, int2 sp, int buf) {
+        if (sp.x > sp.y) return;
+        const int n = min(sp.y - sp.x, W - 1) + 1;
+        // voxel (position p, line L) at ((y - 1) nu + (x - 1)) nv
+        const float *line = g + (rows ? (size_t)(L - 1) * nu + (sp.x - 1) : (size_t)(sp.x - 1) * nu + (L - 1)) * nv;
 #pragma unroll
         for (int i = 0; i < NE; ++i) {
-            const int e = tid + 256 * i;
-            const int j = e / G, gq = e - j * G;
-            pre[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (e < n_el)
-                pre[i] = *reinterpret_cast<const float4 *>(g + base + (size_t)(sp.x + j - 1) * step + z0 + 4 * gq);
+            if (w64 + TL * i >= n * GP) break;
+            if (st_j[i] < n)
+                __builtin_amdgcn_global_load_lds(
+                    (const __attribute__((address_space(1))) void *)(line + st_off[i]),
+                    (__attribute__((address_space(3))) void *)(&seg[buf][sr][0][0] + 4 * (w64 + TL * i)), 16, 0, 0);
         }
     };
-    auto put = [&](int L, int buf) {
-        const int2 sp = spans[L - 1];
-        const int n_el = (min(sp.y - sp.x, W - 1) + 1) * G;
-#pragma unroll
-        for (int i = 0; i < NE; ++i) {
-            const int e = tid + 256 * i;
-            const int j = e / G, gq = e - j * G;
-            if (e < n_el) *reinterpret_cast<float4 *>(&seg[buf][j][4 * gq]) = pre[i];
-        }
+    auto uniform = [](int2 v) {
+        return make_int2(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y));
     };
     // weight of the voxel at position p of line L for this thread's bin (0
     // when it does not contribute), with the forward's float operations
@@ -918,8 +888,8 @@ __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict
         const float uu = lsu - s * (float)x;
         return fmaxf(0.0f, 1.0f - fabsf(uu - fu));
     };
-    // adds the voxel at position p of line L (staged in seg[buf]) with weight w
-    auto add = [&](int L, int p, int buf, const int2 sp, float w) {
+    // adds the voxel at position p of a staged line with weight w
+    auto add = [&](const float (&line)[W][RS], int p, const int2 sp, float w) {
         // staged positions only (a position outside [lo, hi] is outside the
         // mask or past the window's run: weight 0, and a staged value is read)
         int j = p - sp.x;
@@ -928,7 +898,7 @@ __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict
         // (the staged values are finite and the sums never -0, so the result
         // is the same)
         if (out || w == 0.0f) return;
-        const float *v = &seg[buf][j][0];
+        const float *v = &line[j][0];
 #pragma unroll
         for (int gq = 0; gq < G; ++gq) {
             const float4 x4 = *reinterpret_cast<const float4 *>(v + 4 * gq);
@@ -940,7 +910,7 @@ __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict
     };
     // the run's window on line L (first voxel: the estimate, one step down
     // if the voxel before it contributes, one step up if it does not)
-    auto consume = [&](int L, int buf, auto wf) {
+    auto consume = [&](int L, const float (&line)[W][RS], const int2 sp, auto wf) {
         float pa, pb;
         if (rows) {
             const float lsu = su + c * (float)L;
@@ -952,36 +922,46 @@ __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict
             pb = (uhi + bb) * inv;
         }
         const int est = (int)ceilf(fminf(pa, pb));
-        const int2 sp = spans[L - 1];
         if constexpr (INTERP == 1) {
             const int p0 = wf(L, est - 1) != 0.0f ? est - 1 : (wf(L, est) != 0.0f ? est : est + 1);
-            // one window position at a time: 112 instead of 146 registers, four
-            // waves per SIMD (1024^2 x 64 x 900: 11.5 against 12.1 ms)
-#pragma unroll 1
-            for (int i = 0; i < 3; ++i) add(L, p0 + i, buf, sp, wf(L, p0 + i));
+#pragma unroll
+            for (int i = 0; i < 3; ++i) add(line, p0 + i, sp, wf(L, p0 + i));
         } else {
             // the window est .. est + 2 holds the run but for a voxel at one
             // of its ends whose weight is within the estimate's rounding of 0
             // (below 1e-4); the weights are the forward's, so the pair stays
             // an exact transpose up to such terms
-#pragma unroll 1
-            for (int i = 0; i < 3; ++i) add(L, est + i, buf, sp, wf(L, est + i));
+#pragma unroll
+            for (int i = 0; i < 3; ++i) add(line, est + i, sp, wf(L, est + i));
         }
     };
-    if (live(1)) {
-        fetch(1);
-        put(1, 0);
+    // the spans are read two steps ahead of their use
+    int2 cur[R], nxt[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        cur[r] = uniform(spans[r]);
+        nxt[r] = uniform(spans[R + r]);
     }
-    if (nu >= 2 && live(2)) fetch(2);
+    stage(1 + sr, uniform(spans[sr]), 0);
     __syncthreads();
-    for (int L = 1; L <= nu; ++L) {
-        const int buf = (L - 1) & 1;
-        // line L + 1: loaded during the previous line, into the other buffer
-        if (L < nu && live(L + 1)) put(L + 1, buf ^ 1);
-        if (L + 2 <= nu && live(L + 2)) fetch(L + 2);
-        if (active && live(L)) {
-            if constexpr (INTERP == 1) consume(L, buf, weight);
-            else consume(L, buf, hat);
+    for (int L = 1, buf = 0; L <= nu; L += R, buf ^= 1) {
+        int2 far[R], mine = nxt[0];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            far[r] = spans[L - 1 + 2 * R + r];
+            if (sr == r) mine = nxt[r];
+        }
+        stage(L + R + sr, mine, buf ^ 1);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (active && cur[r].x <= cur[r].y) {
+                if constexpr (INTERP == 1) consume(L + r, seg[buf][r], cur[r], weight);
+                else consume(L + r, seg[buf][r], cur[r], hat);
+            }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            cur[r] = nxt[r];
+            nxt[r] = uniform(far[r]);
         }
         __syncthreads();
     }
@@ -990,7 +970,8 @@ __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict
     const float w = wts[idx[k]];
     float *o = out + (size_t)idx[k] * nv * nu + u;
 #pragma unroll
-    for (int z = 0; z < ZT; ++z) o[(size_t)(z0 + z) * nu] = w * acc[z];
+    for (int z = 0; z < ZT; ++z)
+        if (z0 + z < nz4) o[(size_t)(z0 + z) * nu] = w * acc[z];
 }
 
 // Bins 1 and nu - 1 of the linear form, whose weights the hat of
@@ -1720,16 +1701,17 @@ extern "C" int mr_bp_parallel_adjoint(mr_bp_plan *plan, const float *d_grad_volu
     int *d_order = reinterpret_cast<int *>(d_chunks + chunks.size());
     MR_HIP(hipMemcpyAsync(d_chunks, chunks.data(), sizeof(int4) * chunks.size(), hipMemcpyHostToDevice, s));
     MR_HIP(hipMemcpyAsync(d_order, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice, s));
-    // slices per block: the largest of 32, 16, 8, 4 that divides 4*(slices/4)
-    // (64 measured slower at 1024^2 x 64 x 900: 13.0 against 12.0 ms, two
-    // waves per SIMD instead of three)
-    const int zt = nz4 % 32 == 0 ? 32 : (nz4 % 16 == 0 ? 16 : (nz4 % 8 == 0 ? 8 : 4));
-    const int nzs = (int)(nz4 / zt), nbt = (int)((q.width + mr::kAdjNB - 1) / mr::kAdjNB);
+    // slices and lines per step: 32 and 1 where the count is a multiple of 32
+    // (16 and 2: 9.3 against 7.1 ms at 1024^2 x 64 x 900; 32 and 2: 11.1, three
+    // blocks per CU), else 16, 8 or 4 (the last tile may be partial) and 2 (1:
+    // 570 against 500 us at 512^2 x 16 x 360)
+    const int zt = nz4 % 32 == 0 ? 32 : (nz4 > 8 ? 16 : (nz4 > 4 ? 8 : 4));
+    const int nzs = (int)((nz4 + zt - 1) / zt), nbt = (int)((q.width + mr::kAdjNB - 1) / mr::kAdjNB);
     const long total = (long)chunks.size() * nbt * nzs;
     MR_REQUIRE(total < (1L << 31) - 8, "adjoint grid too large");
     const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
     const bool nn = q.interp == MR_INTERP_NEAREST;
-    const size_t dyn = sizeof(int2) * q.width;
+    const size_t dyn = sizeof(int2) * (q.width + 3 * 2);   // 3 R: none beyond the last line
     mr::ProfScope prof("bp_adjoint", s);
     if (!nn) {
         // bins 1 and nu - 1 on the plan's side stream, beside the main kernel
@@ -1747,9 +1729,9 @@ extern "C" int mr_bp_parallel_adjoint(mr_bp_plan *plan, const float *d_grad_volu
         MR_HIP(hipEventRecord(plan->ev_join, plan->side));
     }
 #define MR_ADJ_LAUNCH(I, Z)                                                                                        \
-    hipLaunchKernelGGL((mr::bp_adjoint_kernel<I, Z>), grid, dim3(256), dyn, s, d_grad_volume, d_grad_proj,        \
-                       plan->d_tab, plan->d_mask, plan->d_cmask, plan->d_idx, plan->d_w, d_chunks, d_order,      \
-                       (int)chunks.size(), nbt, nzs, (int)q.width, (int)q.slices)
+    hipLaunchKernelGGL((mr::bp_adjoint_kernel<I, Z, (Z == 32 ? 1 : 2)>), grid, dim3(256), dyn, s, d_grad_volume,   \
+                       d_grad_proj, plan->d_tab, plan->d_mask, plan->d_cmask, plan->d_idx, plan->d_w, d_chunks,    \
+                       d_order, (int)chunks.size(), nbt, nzs, (int)q.width, (int)q.slices, (int)nz4)
     switch (zt) {
     case 32: if (nn) MR_ADJ_LAUNCH(1, 32); else MR_ADJ_LAUNCH(0, 32); break;
     case 16: if (nn) MR_ADJ_LAUNCH(1, 16); else MR_ADJ_LAUNCH(0, 16); break;
