@@ -21,7 +21,6 @@ struct BpArgs {
     int order;           // block -> tile mapping (tile_of_block)
     int ntx, nty, ntz;   // tiles along x, y and slice chunks
     int sw;              // stripe width (tiles) of the XCD-striped order
-    int stage64;         // 1: stage with 64-bit addresses even when 32-bit offsets fit (tests)
     // axis-tilt branch: 0 none, 1 MultiProjBPparallel, 2 MultiProjBP,
     // 3 NearestNeighborBP; centeroffset and centerinc of the block
     int tilt;

@@ -303,11 +303,19 @@ __global__ __launch_bounds__(256) void bp_tilt_kernel(BpArgs a)
 }
 
 // LDS-staged variant.  A block owns a 16 x 16 voxel tile and ZT slices.  For
-// each chunk of KC projections it stages, per projection, the SPAN detector
+// each chunk of projections it stages, per projection, the SPAN detector
 // columns the tile can reach (the tile diagonal spans at most 15*sqrt(2)+2
-// columns, plus one column of rounding margin below) x ZT slices into LDS, then every thread gathers its two columns
-// from LDS with 16-byte reads.  Rows of the staged tile are ZT+4 floats apart,
-// which spreads 16 distinct columns over distinct LDS banks.
+// columns, plus one column of rounding margin below) x ZT slices into LDS, then
+// every thread gathers its two columns from LDS with 16-byte reads.  Rows of
+// the staged tile are ZT+4 floats apart, which spreads 16 distinct columns over
+// distinct LDS banks.  Two buffers of C projections (KC of them where two fit
+// beside enough blocks, else KC / 2): direct loads fill one while the other is
+// summed, one barrier per chunk; the lowest columns of 64 projections are
+// computed at once, one per lane.  (Staged through registers between two
+// barriers, lowest columns in LDS: exact 1024^2 x 32 x 625 2.06 against 1.89 ms,
+// nearest neighbour 512^2 x 64 x 200 0.224 against 0.171, tilted 1024^2 x 64 x 300
+// 2.27 against 2.11.)  Bound by the LDS reads, 8 bytes per voxel, slice and
+// projection: 1.8 of the 1.89 ms at 128 bytes per cycle and CU.
 // EXACT = true keeps the reference's float operation order per voxel
 // (bit-identical); EXACT = false folds the interpolation into two FMAs.
 constexpr int kBpSpan = 26;
@@ -324,9 +332,13 @@ constexpr int kBpSpan = 26;
 // as in bp_tilt_kernel (1 MultiProjBPparallel, 2 MultiProjBP, 3
 // NearestNeighborBP): the detector position shifted by centeroffset and the
 // interpolation weight recomputed per slice group.
+template <int ZT, int KC> struct BpStage {
+    static constexpr int C = ZT == 32 || KC <= 4 ? KC : KC / 2;
+    float buf[2][C][kBpSpan][ZT + 4];
+};
+
 template <int ZT, int INTERP, bool EXACT, int KC, int PIPE, int TILT = 0>
-__device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int bz,
-                                            float (&sm)[KC][kBpSpan][ZT + 4], int (&sb0)[KC])
+__device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int bz, BpStage<ZT, KC> &lds)
 {
     static_assert(TILT == 0 || (PIPE == 0 && EXACT), "the tilt branches run on the reference-order, rolled path");
     static_assert(TILT != 3 || INTERP == 1, "NearestNeighborBP's tilt branch is the nearest-neighbour form");
@@ -354,97 +366,78 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
     if (any_inside && zl > 0) {
         const float yf = (float)(y + 1), xf = (float)(x + 1);
         const int num2 = a.nu - 2;
-        // Staging: element e = threadIdx.x + 256 i of a chunk is (projection
-        // kk, column b, slice group q).  Its LDS slot and its byte offset in
-        // the chunk (less the column term) do not change between chunks, so
-        // they are computed once here; a chunk then costs one multiply-add
-        // per element.  Loads go through a buffer resource over the chunk:
-        // slices at or beyond 4*(nv/4) get an offset past its end and read as
-        // zeros (the accumulation below runs over every group of the tile and
-        // leaves them unchanged), and columns past the detector edge, which no
-        // voxel reads, stay inside the buffer or read as zeros.  Chunks too
-        // large for 32-bit offsets take the general loop.
-        constexpr int NE = (KC * SPAN * G + 255) / 256;
+        // Staging: wave w takes projections w, w + 4, ... of a chunk, each as
+        // 16-byte chunks of SPAN columns from the lowest one any voxel of the
+        // tile reaches: G of a column's slices and one lane whose offset lies
+        // past the buffer (so that columns lie ZT + 4 floats apart), as do
+        // slices at or beyond 4*(nv/4), which read as zeros.  Columns past the
+        // detector edge, which no voxel reads, stay inside the buffer or read
+        // as zeros.
+        constexpr int C = BpStage<ZT, KC>::C, GP = G + 1, NE = (SPAN * GP + 63) / 64;
+        static_assert(64 % C == 0, "a chunk lies in one group of 64 projections");
+        const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         const int vpad4 = 4 * a.vpad;
-        const bool off32 = !a.stage64 && (long)KC * (a.nu + SPAN) * vpad4 < 0x7FFFFFF0L;
-        int st_kk[NE], st_b[NE], st_lds[NE];
         unsigned st_off[NE];
 #pragma unroll
         for (int i = 0; i < NE; ++i) {
-            const int e = (int)threadIdx.x + 256 * i;
-            const int kk = e / (SPAN * G);
-            const int r = e - kk * SPAN * G;
-            const int b = r / G, q = r - b * G;
-            st_kk[i] = e < KC * SPAN * G ? kk : KC;
-            st_b[i] = b;
-            st_lds[i] = (kk * SPAN + b) * RS + 4 * q;
-            // unsigned: only used when the chunk fits 32-bit offsets (off32)
-            st_off[i] = z0 + 4 * q < a.nz4
-                            ? (unsigned)kk * (unsigned)a.nu * (unsigned)vpad4 + 4u * (unsigned)(z0 + 4 * q)
-                            : 0x80000000u;
+            const int b = (lane + 64 * i) / GP, q = (lane + 64 * i) - b * GP;
+            st_off[i] = q < G && z0 + 4 * q < a.nz4 ? (unsigned)b * (unsigned)vpad4 + 16u * (unsigned)q : 0x80000000u;
         }
-        float *smf = &sm[0][0][0];
-        for (int kb = 0; kb < a.nk; kb += KC) {
-            const int kc = min(KC, a.nk - kb);
-            if (threadIdx.x < kc) {
-                // lowest detector column any voxel of the tile reaches
-                const float4 t = a.tab[kb + threadIdx.x];
-                const float ya = (float)(y0 + 1), yb = (float)(y0 + T);
-                const float xa = (float)(x0 + 1), xb = (float)(x0 + T);
-                int n0;
-                if constexpr (TILT == 1) {
-                    const float la = (t.x + t.y * ya) - a.tilt_co, lb = (t.x + t.y * yb) - a.tilt_co;
-                    n0 = min(min((int)(la - t.z * xa), (int)(la - t.z * xb)),
-                             min((int)(lb - t.z * xa), (int)(lb - t.z * xb)));
-                } else if constexpr (TILT >= 2) {
-                    const float la = t.x + t.y * ya, lb = t.x + t.y * yb, co = a.tilt_co;
-                    n0 = min(min((int)((la - t.z * xa) - co), (int)((la - t.z * xb) - co)),
-                             min((int)((lb - t.z * xa) - co), (int)((lb - t.z * xb) - co)));
-                } else {
-                    const float la = t.x + t.y * ya, lb = t.x + t.y * yb;
-                    n0 = min(min((int)(la - t.z * xa), (int)(la - t.z * xb)),
-                             min((int)(lb - t.z * xa), (int)(lb - t.z * xb)));
-                }
-                // one bin of margin: an interior voxel may round one ulp below a
-                // corner and truncate to the bin below
-                sb0[threadIdx.x] = max(n0 - 1, 0);
+        // lowest column of projection 64 j + lane: one bin of margin, an interior
+        // voxel may round one ulp below a corner and truncate to the bin below
+        auto lowest = [&](int kb) {
+            const float4 t = a.tab[min(kb + lane, a.nk - 1)];
+            const float ya = (float)(y0 + 1), yb = (float)(y0 + T);
+            const float xa = (float)(x0 + 1), xb = (float)(x0 + T);
+            int n0;
+            if constexpr (TILT == 1) {
+                const float la = (t.x + t.y * ya) - a.tilt_co, lb = (t.x + t.y * yb) - a.tilt_co;
+                n0 = min(min((int)(la - t.z * xa), (int)(la - t.z * xb)),
+                         min((int)(lb - t.z * xa), (int)(lb - t.z * xb)));
+            } else if constexpr (TILT >= 2) {
+                const float la = t.x + t.y * ya, lb = t.x + t.y * yb, co = a.tilt_co;
+                n0 = min(min((int)((la - t.z * xa) - co), (int)((la - t.z * xb) - co)),
+                         min((int)((lb - t.z * xa) - co), (int)((lb - t.z * xb) - co)));
+            } else {
+                const float la = t.x + t.y * ya, lb = t.x + t.y * yb;
+                n0 = min(min((int)(la - t.z * xa), (int)(la - t.z * xb)),
+                         min((int)(lb - t.z * xa), (int)(lb - t.z * xb)));
             }
-            __syncthreads();
-            if (off32) {
-                const float *cb = a.sino + (size_t)kb * a.nu * a.vpad;
-                const long rem = (long)(a.nk - kb) * a.nu * vpad4;
-                const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                    (void *)cb, (short)0, (int)min(rem, 0x7FFFFFF0L), 0x00020000);
-                // all loads first, then the LDS writes, so the loads are in
-                // flight together; elements of absent projections (last
-                // chunk) load zeros from an offset past the buffer, and any
-                // offset is safe with a buffer resource
-                float4 v[NE];
+            return max(n0 - 1, 0);
+        };
+        const size_t row = (size_t)a.nu * a.vpad;
+        auto stage = [&](int kb, int low, float (&dst)[C][SPAN][RS]) {
+            (void)wv;
+            (void)row;
+#if defined(__HIP_DEVICE_COMPILE__)   // (the host pass rejects a second use of a body with these builtins)
 #pragma unroll
-                for (int i = 0; i < NE; ++i) {
-                    const unsigned col = (unsigned)(sb0[min(st_kk[i], KC - 1)] + st_b[i]);
-                    const unsigned off = st_kk[i] < kc ? col * (unsigned)vpad4 + st_off[i] : 0x80000000u;
-                    // the whole 16-byte result is reinterpreted: indexing its
-                    // elements makes this compiler load one dword only
-                    v[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
-                }
+            for (int kk = wv; kk < C; kk += 4) {
+                if (kb + kk >= a.nk) break;
+                const int n0 = __builtin_amdgcn_readlane(low, (kb + kk) & 63);
+                const size_t at = (size_t)(kb + kk) * row + (size_t)n0 * a.vpad;
+                const long left = 4 * ((long)((size_t)a.nk * row) - (long)at);
+                const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                    (void *)(a.sino + at + z0), (short)0, (int)max(0L, min(left - 4 * z0, 0x7FFFFFF0L)), 0x00020000);
 #pragma unroll
                 for (int i = 0; i < NE; ++i)
-                    if (st_kk[i] < KC) *reinterpret_cast<float4 *>(smf + st_lds[i]) = v[i];
-            } else {
-                for (int e = threadIdx.x; e < kc * SPAN * G; e += 256) {
-                    const int kk = e / (SPAN * G);
-                    const int r = e - kk * SPAN * G;
-                    const int b = r / G, q = r - b * G;
-                    const int col = sb0[kk] + b;
-                    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    if (col < a.nu && z0 + 4 * q < a.nz4)
-                        v = *reinterpret_cast<const float4 *>(
-                            a.sino + ((size_t)(kb + kk) * a.nu + col) * a.vpad + z0 + 4 * q);
-                    *reinterpret_cast<float4 *>(&sm[kk][b][4 * q]) = v;
-                }
+                    if (lane + 64 * i < SPAN * GP)
+                        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                            rs, (__attribute__((address_space(3))) void *)(&dst[kk][0][0] + 256 * i), 16, st_off[i], 0,
+                            0, 0);
             }
-            __syncthreads();
+#endif
+        };
+        int low = lowest(0), low_next = low;
+        stage(0, low, lds.buf[0]);
+        __syncthreads();
+        for (int kb = 0, buf = 0; kb < a.nk; kb += C, buf ^= 1) {
+            const int kc = min(C, a.nk - kb);
+            const float (&sm)[C][SPAN][RS] = lds.buf[buf];
+            // the next chunk's loads are in flight while this one is summed
+            if (kb + C < a.nk) {
+                if (((kb + C) & 63) == 0) low_next = lowest(kb + C);
+                stage(kb + C, low_next, lds.buf[buf ^ 1]);
+            }
             if constexpr (PIPE == 0) {
             if (inside) {
                 for (int kk = 0; kk < kc; ++kk) {
@@ -462,7 +455,7 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
                     }
                     const int n = (int)u;
                     if (n < 0 || n > num2) continue;
-                    const int loc = min(max(n - sb0[kk], 0), SPAN - 2);
+                    const int loc = min(max(n - __builtin_amdgcn_readlane(low, (kb + kk) & 63), 0), SPAN - 2);
                     const float *A = &sm[kk][loc][0];
                     if constexpr (TILT == 1 || TILT == 2) {
                         // per slice group g (from the block's first slice): weight
@@ -538,11 +531,11 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
                 // the chunk's staging offsets in scalar registers; the
                 // projection loop is unrolled so neighbouring projections'
                 // LDS reads and FMAs interleave
-                int sbr[KC];
+                int sbr[C];
 #pragma unroll
-                for (int q = 0; q < KC; ++q) sbr[q] = __builtin_amdgcn_readfirstlane(sb0[q]);
+                for (int q = 0; q < C; ++q) sbr[q] = __builtin_amdgcn_readlane(low, (kb + q) & 63);
 #pragma unroll
-                for (int kk = 0; kk < KC; ++kk) {
+                for (int kk = 0; kk < C; ++kk) {
                     if (kk >= kc) break;
                     const float4 t = tab_entry(a.tab, kb + kk);
                     const float lsu = t.x + t.y * yf;
@@ -584,6 +577,7 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
                 }
             }
             }
+            low = low_next;
             __syncthreads();
         }
     }
@@ -603,23 +597,21 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
 template <int ZT, int INTERP, bool EXACT, int KC, int PIPE>
 __global__ __launch_bounds__(256) void bp_lds_kernel(BpArgs a)
 {
-    __shared__ float sm[KC][kBpSpan][ZT + 4];
-    __shared__ int sb0[KC];
+    __shared__ __align__(16) BpStage<ZT, KC> lds;
     if (a.gate && *a.gate == 0) return;
     int bx, by, bz;
     if (!tile_of_block(a, bx, by, bz)) return;
-    bp_lds_tile<ZT, INTERP, EXACT, KC, PIPE>(a, bx, by, bz, sm, sb0);
+    bp_lds_tile<ZT, INTERP, EXACT, KC, PIPE>(a, bx, by, bz, lds);
 }
 
 // The tilt branches on the same tiles (reference order, rolled loop).
 template <int ZT, int INTERP, int KC, int TILT>
 __global__ __launch_bounds__(256) void bp_lds_tilt_kernel(BpArgs a)
 {
-    __shared__ float sm[KC][kBpSpan][ZT + 4];
-    __shared__ int sb0[KC];
+    __shared__ __align__(16) BpStage<ZT, KC> lds;
     int bx, by, bz;
     if (!tile_of_block(a, bx, by, bz)) return;
-    bp_lds_tile<ZT, INTERP, true, KC, 0, TILT>(a, bx, by, bz, sm, sb0);
+    bp_lds_tile<ZT, INTERP, true, KC, 0, TILT>(a, bx, by, bz, lds);
 }
 
 // Persistent batched back-projection: a grid sized to the device (every
@@ -642,8 +634,7 @@ __global__ __launch_bounds__(256) void bp_batch_kernel(const BpArgs *__restrict_
         for (int i = threadIdx.x; i < n_stacks; i += 256) any |= flags[i];
         if (!__syncthreads_or(any)) return;
     }
-    __shared__ float sm[KC][kBpSpan][ZT + 4];
-    __shared__ int sb0[KC];
+    __shared__ __align__(16) BpStage<ZT, KC> lds;
     __shared__ int item;
     int part = (int)(blockIdx.x & 7);
     for (;;) {
@@ -668,8 +659,8 @@ __global__ __launch_bounds__(256) void bp_batch_kernel(const BpArgs *__restrict_
         const int4 w = items[it];
         if (flags && !flags[w.x]) continue;
         const BpArgs a = stacks[w.x];
-        bp_lds_tile<ZT, INTERP, EXACT, KC, ((ZT == 32 && KC == 4) || (ZT == 16 && KC == 8)) ? 1 : 0>(
-            a, w.y, w.z, w.w, sm, sb0);
+        constexpr int PIPE = (ZT == 32 && KC == 4) || (ZT == 16 && KC == 8) ? 1 : 0;
+        bp_lds_tile<ZT, INTERP, EXACT, KC, PIPE>(a, w.y, w.z, w.w, lds);
         __syncthreads();
     }
 }
@@ -1116,33 +1107,31 @@ static void lds_shape(int nu, int nv, int &zt, int &kc, int &pipe)
     pipe = zt == 8 ? 0 : 1;
 }
 
-// The same for nk projections.  A block's chunks follow one another (barrier,
-// table entries, loads, barrier, sums), and one or two waves per SIMD neither
-// cover those latencies nor issue at full rate (one: 8 cycles per instruction,
-// four: 2.4), so a grid of few blocks takes thinner slice tiles: 4 slices with
-// chunks of 32 while that makes at most 5 blocks per CU, else 8 slices with
-// chunks of 8 where the shape above has fewer than 4 blocks per CU or fewer
-// than 16 slices.  The positions and weights, computed once per tile, are then
-// computed more often.  Exact, in microseconds (shape above, 4, 8 slices):
-// 256^2 x 16 x 180: 71, 48, 55; 128^2 x 16 x 180: 87, 41, 53; 256^2 x 8 x 180:
-// 57, 41, 53; 300^2 x 10 x 700: 207, 166, 196; 256^2 x 24 x 360 (1536 blocks of
-// 4 slices): 145, 150, 108; 400^2 x 16 x 360: 153, 161, 129; 512^2 x 8 x 360:
-// 136, 150, 112; 512^2 x 16 x 360 (1024 blocks): 184, 243, 206.  Below 8 slices
-// the unrolled chunks would add zeros (1024^2 x 4 x 400: 302 above, 363 with 8).
-// Fewer than 64 projections are a few chunks whichever way and keep the shape
-// above.
+// The same for nk projections.  One or two waves per SIMD neither cover the
+// latencies of a block's chunks nor issue at full rate (one wave: 8 cycles per
+// instruction, four: 2.4), so a grid of few blocks takes thinner slice tiles,
+// unrolled and with chunks of 16: 4 slices where 8 would make at most one block
+// per CU, else 8 where the shape above has fewer than 4 blocks per CU or fewer
+// than 16 slices (not below 8 slices: the unrolled tile would add zeros).  The
+// positions and weights, computed once per tile, are then computed more often.
+// Exact, in microseconds (shape above, 4, 8 slices): 128^2 x 16 x 180: 81, 38,
+// 46; 256^2 x 8 x 180: 58, 38, 47; 256^2 x 16 x 180: 67, 53, 49; 400^2 x 16 x
+// 360: 143, 168, 130; 300^2 x 10 x 700: 222, 190, 183; 512^2 x 8 x 360: 129,
+// 160, 113; 512^2 x 16 x 360 (1024 blocks): 190, -, 206; 1024^2 x 4 x 200: 156,
+// 153, 187.  Fewer than 32 projections are two chunks whichever way and keep
+// the shape above.
 static void lds_shape_nk(int nu, int nv, int nk, int &zt, int &kc, int &pipe)
 {
     lds_shape(nu, nv, zt, kc, pipe);
     const long tiles = (long)((nu + 15) / 16) * ((nu + 15) / 16);
-    if (nk < 64 || zt == 32) return;
-    if (tiles * ((nv + 3) / 4) <= 1280 && (nv >= 8 || tiles <= 512)) {
+    if (nk < 32 || zt == 32) return;
+    if (tiles * ((nv + 7) / 8) <= 256) {
         zt = 4;
-        kc = 32;
-        pipe = 0;
+        kc = 16;
+        pipe = 1;
     } else if (nv >= 8 && (zt == 8 || tiles * ((nv + 15) / 16) < 1024)) {
         zt = 8;
-        kc = 8;
+        kc = 16;
         pipe = 1;
     }
 }
@@ -1187,8 +1176,8 @@ int run_bp(const BpArgs &a, int interp, int impl, int exact, hipStream_t s)
     lds_shape_nk(a.nu, a.nv, a.nk, zt, kc, pipe);
     if (zt == 32) return launch_bp_lds_mode<32, 4, 1>(a, interp, exact, s);
     if (zt == 16) return launch_bp_lds_mode<16, 8, 1>(a, interp, exact, s);
-    if (zt == 4) return launch_bp_lds_mode<4, 32, 0>(a, interp, exact, s);
-    if (pipe) return launch_bp_lds_mode<8, 8, 1>(a, interp, exact, s);
+    if (zt == 4) return launch_bp_lds_mode<4, 16, 1>(a, interp, exact, s);
+    if (pipe) return launch_bp_lds_mode<8, 16, 1>(a, interp, exact, s);
     return launch_bp_lds_mode<8, 16, 0>(a, interp, exact, s);
 }
 
@@ -1238,7 +1227,7 @@ struct mr_bp_plan {
     int *d_idx = nullptr;
     float *d_w = nullptr;
     int impl = 1;  // 1 LDS-staged kernel, 0 direct-gather kernel
-    int stage64 = 0;  // 1: 64-bit staging addresses (MR_BP_STAGE64 debug override)
+    int stage64 = 0;  // 1: no matrix-core form (MR_BP_STAGE64 debug override)
     size_t loaded_n = 0, loaded_nk = 0;   // projections / used projections of the resident tables
     bool loaded = false;
     void *d_adj = nullptr;                // adjoint chunks (int4) and projection order (int)
@@ -1363,9 +1352,8 @@ extern "C" int mr_bp_plan_create(mr_bp_plan **plan, const mr_bp_params *params)
     // MultiProjBP's B-column offset only differs from the padded column when
     // slices % 4 != 0; that case stays on the direct-gather kernel.
     p->impl = (q.multiprojbp && (q.slices & 3)) ? 0 : 1;
-    // debug override, read once per plan: MR_BP_STAGE64=1 makes the LDS
-    // kernel stage through 64-bit addresses, the path that chunks too large
-    // for 32-bit buffer offsets take (tested bit-identical to the default)
+    // debug override, read once per plan: MR_BP_STAGE64=1 keeps the fused form on
+    // the vector kernel (whose staging takes 64-bit addresses at every size)
     if (const char *e = std::getenv("MR_BP_STAGE64")) p->stage64 = std::atoi(e) == 1 ? 1 : 0;
     mr::circle_mask(q.width, q.width, q.use_roi != 0, q.roi, false, p->first, p->second,
                     q.correct_tilt ? mr::tilt_mask_shrink(q.tilt_angle, q.tilt_rows) : 0.0f);
@@ -1524,7 +1512,6 @@ int bp_enqueue(mr_bp_plan *plan, const float *d_proj, float *d_volume, int accum
     a.nz4 = (int)((q.slices / 4) * 4);
     a.bstride = q.multiprojbp ? a.nz4 : (int)plan->vpad;
     a.accumulate = accumulate ? 1 : 0;
-    a.stage64 = plan->stage64;
     a.gate = flag;
     a.tilt = plan->tilt;
     if (plan->tilt) mr::bp_tilt_terms(q.tilt_angle, q.tilt_pivot, plan->tilt_row0, a.tilt_co, a.tilt_ci);

@@ -1,10 +1,10 @@
 """Small parallel-beam grids: 4- and 8-slice tiles.
 
-With 64 projections or more, a grid of few blocks takes tiles of 4 slices
-(chunks of 32 projections) or 8 (chunks of 8).  Sizes on both sides of each line
-of the rule, with remainders in slices, projections and tiles, against the
-oracle: bit for bit in reference order (both interpolations), relRMSE <= 1e-6 in
-fused mode; and the kernel that the plan reports before and after the tables.
+With 32 projections or more, a grid of few blocks takes tiles of 4 or 8 slices
+(unrolled, chunks of 16 projections).  Sizes on both sides of each line of the
+rule, with remainders in slices, projections and tiles, against the oracle: bit
+for bit in reference order (both interpolations), relRMSE <= 1e-6 in fused mode;
+and the kernel that the plan reports before and after the tables.
 """
 import numpy as np
 import pytest
@@ -15,15 +15,16 @@ from conftest import rel_err
 pytestmark = pytest.mark.gpu
 
 # width, slices, projections, template arguments after the plan has its tables
-SHAPES = [(64, 1, 64, "4,0,{},32,0"),
-          (100, 18, 71, "4,0,{},32,0"),
-          (64, 13, 63, "8,0,{},16,0"),
-          (250, 20, 65, "4,0,{},32,0"),
-          (250, 21, 66, "8,0,{},8,1"),
-          (300, 15, 80, "8,0,{},8,1"),
-          (336, 17, 64, "8,0,{},8,1"),
+SHAPES = [(64, 1, 32, "4,0,{},16,1"),
+          (100, 18, 71, "4,0,{},16,1"),
+          (64, 13, 31, "8,0,{},16,0"),
+          (256, 8, 65, "4,0,{},16,1"),
+          (256, 9, 65, "8,0,{},16,1"),
+          (250, 21, 66, "8,0,{},16,1"),
+          (300, 15, 129, "8,0,{},16,1"),
+          (336, 17, 64, "8,0,{},16,1"),
           (500, 7, 70, "8,0,{},16,0"),
-          (500, 8, 70, "8,0,{},8,1"),
+          (500, 8, 70, "8,0,{},16,1"),
           (513, 16, 66, "16,0,{},8,1")]
 
 
