@@ -466,19 +466,23 @@ __global__ __launch_bounds__(256) void joseph_adjoint_kernel(JosephArgs a)
 }
 
 // LDS-staged adjoint: the structure of the parallel back-projector's tiled
-// kernel (16 x 16 voxel tile, ZT slices, KC angles staged per chunk, the
-// XCD-striped tile order) with the Joseph kernel K as weights.  For each
-// angle the tile stages the SPAN detector bins from floor(u) of its lowest
-// corner; bins outside [0, n_det) are staged as zeros, which is where the
-// direct kernel's clamped loads have weight zero.
+// kernel (16 x 16 voxel tile, ZT slices, C angles staged per chunk by direct
+// loads into one of two buffers while the other is summed, the XCD-striped tile
+// order) with the Joseph kernel K as weights.  For each angle the tile stages
+// the SPAN detector bins from floor(u) of its lowest corner, one bin of rounding
+// margin below; bins outside [0, n_det) are staged as zeros, which is where the
+// direct kernel's clamped loads have weight zero, and so are slices past the
+// last.  Bound by the LDS reads.  (Staged between two barriers per chunk:
+// 512^2 x 16 x 360 207 against 166 us, 512^2 x 32 x 360 358 against 272, 1024^2 x
+// 64 x 200 1.32 against 1.16 ms.)
 constexpr int kJSpan = 26;
 
-template <int ZT, int KC>
+template <int ZT, int C>
 __global__ __launch_bounds__(256) void joseph_adjoint_lds_kernel(JosephArgs a, int ntx, int nty, int ntz)
 {
-    constexpr int T = 16, SPAN = kJSpan, G = ZT / 4;
-    __shared__ float sm[KC][SPAN][ZT + 4];
-    __shared__ int sb0[KC];
+    constexpr int T = 16, SPAN = kJSpan, G = ZT / 4, GP = G + 1, NE = (SPAN * GP + 63) / 64;
+    static_assert(64 % C == 0, "a chunk lies in one group of 64 angles");
+    __shared__ __align__(16) float sm[2][C][SPAN][4 * GP];
     // block -> tile: XCD c (= block % 8) takes the c-th eighth of the tiles in
     // slice-chunk, 4-column stripe, row order
     const int n = ntx * nty * ntz;
@@ -505,30 +509,54 @@ __global__ __launch_bounds__(256) void joseph_adjoint_lds_kernel(JosephArgs a, i
 #pragma unroll
     for (int z = 0; z < ZT; ++z) acc[z] = 0.0f;
     const float xf = (float)(x + 1), yf = (float)(y + 1);
-    for (int kb = 0; kb < a.na; kb += KC) {
-        const int kc = min(KC, a.na - kb);
-        if (threadIdx.x < kc) {
-            const float4 t = a.tab[kb + threadIdx.x];
-            const float ya = (float)(y0 + 1), yb = (float)(y0 + T);
-            const float xa = (float)(x0 + 1), xb = (float)(x0 + T);
-            const float la = t.x + t.y * ya, lb = t.x + t.y * yb;
-            const float umin = fminf(fminf(la - t.z * xa, la - t.z * xb), fminf(lb - t.z * xa, lb - t.z * xb));
-            sb0[threadIdx.x] = (int)floorf(umin) - 1;   // one bin of rounding margin
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // wave w stages angles w, w + 4, ... of a chunk in 16-byte chunks: G of a
+    // bin's slices and one lane whose offset lies past the buffer
+    int st_b[NE];
+    unsigned st_off[NE];
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+        const int b = (lane + 64 * i) / GP, g = (lane + 64 * i) - b * GP;
+        st_b[i] = b;
+        st_off[i] = g < G && z0 + 4 * g < a.nz ? 4u * (unsigned)b * (unsigned)a.nz + 16u * (unsigned)g : 0x80000000u;
+    }
+    // lowest bin of angle 64 j + lane
+    auto lowest = [&](int kb) {
+        const float4 t = a.tab[min(kb + lane, a.na - 1)];
+        const float ya = (float)(y0 + 1), yb = (float)(y0 + T);
+        const float xa = (float)(x0 + 1), xb = (float)(x0 + T);
+        const float la = t.x + t.y * ya, lb = t.x + t.y * yb;
+        const float umin = fminf(fminf(la - t.z * xa, la - t.z * xb), fminf(lb - t.z * xa, lb - t.z * xb));
+        return (int)floorf(umin) - 1;
+    };
+    auto stage = [&](int kb, int low, float (&dst)[C][SPAN][4 * GP]) {
+#pragma unroll
+        for (int kk = wv; kk < C; kk += 4) {
+            if (kb + kk >= a.na) break;
+            const int n0 = __builtin_amdgcn_readlane(low, (kb + kk) & 63);
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                (void *)(a.src + (((long)(kb + kk) * a.nd + n0) * a.nz + z0)), (short)0, 0x7FFFFFFF, 0x00020000);
+#pragma unroll
+            for (int i = 0; i < NE; ++i) {
+                const unsigned off = (unsigned)(n0 + st_b[i]) < (unsigned)a.nd ? st_off[i] : 0x80000000u;
+                if (lane + 64 * i < SPAN * GP)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                        rs, (__attribute__((address_space(3))) void *)(&dst[kk][0][0] + 256 * i), 16, off, 0, 0, 0);
+            }
         }
-        __syncthreads();
-        for (int e = threadIdx.x; e < kc * SPAN * G; e += 256) {
-            const int kk = e / (SPAN * G);
-            const int rr = e - kk * SPAN * G;
-            const int bb = rr / G, g = rr - bb * G;
-            const int col = sb0[kk] + bb;
-            float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (col >= 0 && col < a.nd && z0 + 4 * g < a.nz)
-                v = *reinterpret_cast<const float4 *>(a.src + ((size_t)(kb + kk) * a.nd + col) * a.nz + z0 + 4 * g);
-            *reinterpret_cast<float4 *>(&sm[kk][bb][4 * g]) = v;
+    };
+    int low = lowest(0), low_next = low;
+    stage(0, low, sm[0]);
+    __syncthreads();
+    for (int kb = 0, buf = 0; kb < a.na; kb += C, buf ^= 1) {
+        if (kb + C < a.na) {
+            if (((kb + C) & 63) == 0) low_next = lowest(kb + C);
+            stage(kb + C, low_next, sm[buf ^ 1]);
         }
-        __syncthreads();
         if (in_vol) {
-            for (int kk = 0; kk < kc; ++kk) {
+#pragma unroll
+            for (int kk = 0; kk < C; ++kk) {
+                if (kb + kk >= a.na) break;
                 const float4 t = tab_entry(a.tab, kb + kk);
                 const float u = (t.x + t.y * yf) - t.z * xf;
                 const float fl = floorf(u);
@@ -537,8 +565,8 @@ __global__ __launch_bounds__(256) void joseph_adjoint_lds_kernel(JosephArgs a, i
                 const float inv_m = t.w;
                 const float w1 = fmaxf(0.0f, 1.0f - f * inv_m) * inv_m;
                 const float w2 = fmaxf(0.0f, 1.0f - (1.0f - f) * inv_m) * inv_m;
-                const int loc = min(max(n1 - sb0[kk], 0), SPAN - 2);
-                const float *A = &sm[kk][loc][0];
+                const int loc = min(max(n1 - __builtin_amdgcn_readlane(low, (kb + kk) & 63), 0), SPAN - 2);
+                const float *A = &sm[buf][kk][loc][0];
                 const float *B = A + (ZT + 4);
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
@@ -551,6 +579,7 @@ __global__ __launch_bounds__(256) void joseph_adjoint_lds_kernel(JosephArgs a, i
                 }
             }
         }
+        low = low_next;
         __syncthreads();
     }
     if (!in_vol) return;
@@ -745,7 +774,7 @@ int joseph_launch(const mr_joseph_geom *g, const float *src, float *dst, const J
         // slices, else 16 (a rest is staged as zeros).  Slice counts that are not
         // a multiple of 16 take the voxel-driven kernel, which gives the same
         // bits, below 512 tiles: 128^2 x 24 x 60 (128 tiles) 18 against 28 us,
-        // 300^2 x 20 x 200 (722) 125 against 101, 700^2 x 8 x 200 220 against 112.
+        // 300^2 x 20 x 200 (722) 125 against 80, 700^2 x 8 x 200 220 against 103.
         const int zt = g->nz % 32 == 0 ? 32 : (g->nz > 8 ? 16 : 8);
         const int ntx = (int)((g->nx + 15) / 16), ntz = (int)((g->nz + zt - 1) / zt);
         const long nt = (long)ntx * ntx * ntz;
@@ -757,9 +786,9 @@ int joseph_launch(const mr_joseph_geom *g, const float *src, float *dst, const J
         } else if (zt == 32) {
             hipLaunchKernelGGL((mr::joseph_adjoint_lds_kernel<32, 4>), grid, dim3(256), 0, s, a, ntx, ntx, ntz);
         } else if (zt == 16) {
-            hipLaunchKernelGGL((mr::joseph_adjoint_lds_kernel<16, 8>), grid, dim3(256), 0, s, a, ntx, ntx, ntz);
+            hipLaunchKernelGGL((mr::joseph_adjoint_lds_kernel<16, 4>), grid, dim3(256), 0, s, a, ntx, ntx, ntz);
         } else {
-            hipLaunchKernelGGL((mr::joseph_adjoint_lds_kernel<8, 16>), grid, dim3(256), 0, s, a, ntx, ntx, ntz);
+            hipLaunchKernelGGL((mr::joseph_adjoint_lds_kernel<8, 8>), grid, dim3(256), 0, s, a, ntx, ntx, ntz);
         }
     }
     MR_HIP(hipGetLastError());
