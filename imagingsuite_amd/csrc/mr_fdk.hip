@@ -910,7 +910,6 @@ extern "C" int mr_fdk_plan_create(mr_fdk_plan **plan, const mr_fdk_params *param
         }
     }
     std::vector<float> tw = mr::make_twiddles(P);
-    ramp = mr::spectrum_order(ramp);
     hipError_t e = hipMalloc(&p->d_mask, sizeof(int2) * p->nx);
     if (e == hipSuccess) e = hipMalloc(&p->d_hs, sizeof(float) * P);
     if (e == hipSuccess) e = hipMalloc(&p->d_tw, sizeof(float2) * P);

@@ -1,55 +1,18 @@
-// LDS-resident FFT filter of one complex line of compile-time length P, shared
-// by the parallel-beam and the FDK ramp filters: forward transform, product
-// with a real spectrum, inverse transform.
+// LDS-resident Stockham FFT for one complex line of compile-time length P,
+// shared by the parallel-beam and the FDK ramp filters.
 //
-// Radix-8 stages, each in place: a thread reads eight points of the line into
-// registers and writes its results to the same eight places.  The forward
-// stages decimate in frequency (span P, P/8, ...), the inverse ones in time
-// (back up), so the spectrum is met in digit-reversed order, where its product
-// and the stages on either side of it are one pass over registers: no
-// reordering, and one exchange through LDS per stage boundary.  The line's
-// remaining factor 2 or 4 is that middle stage.
-//
-// A stage of span N works on runs of N points by N / 8 consecutive threads, so
-// from span 512 down a run stays within one wave and needs no block barrier:
-// P = 4096 has two (after the first and before the last stage).
-//
-// Bank conflicts: point i lies at i ^ ((i >> 3) & 31).  In every stage the five
-// index bits that vary over 32 consecutive lanes (bits 0 .. 4 for a stride of
-// 32 or more, the low bits and those above the three stage bits for smaller
-// ones, bits 3 .. 7 in the middle stage) then reach all 32 pairs of banks.
-//
-// Twiddles: powers 1, 2 and 4 of each stage are table entries (in double on the
-// host, coalesced loads ahead of the stage's exchange), the others products of
-// them.  A filtered row is small beside its input where a ramp meets smooth
-// data, so the twiddles' errors count: with all powers made from the first the
-// result is 1.6 to 2 times further from double than with these (rows of 2048:
-// 2.1e-5 against 1.2e-5 of the result, all seven from a table 1.1e-5).
+// The line lives in LDS as float2[P].  Passes are radix-4 (plus one radix-2
+// pass first when log2 P is odd); every pass reads its butterfly inputs into
+// registers, synchronises, and writes the outputs back in natural (Stockham
+// autosort) order, so no bit reversal is needed.  Twiddles come from a
+// P-entry table tw[k] = exp(-2 pi i k / P) computed in double on the host.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
-#include <type_traits>
-
 namespace mr {
 
 constexpr int ilog2c(int v) { return v <= 1 ? 0 : 1 + ilog2c(v >> 1); }
-
-// Stages of the P-point line: kFftStages(P) of radix 8 with a twiddle, then the
-// middle stage of radix fft_mid(P).
-constexpr int fft_mid(int P) { return ilog2c(P) % 3 == 0 ? 8 : 1 << (ilog2c(P) % 3); }
-constexpr int fft_stages(int P) { return ilog2c(P / fft_mid(P)) / 3; }
-// Table offset of stage s: spans P, P/8, ... with 3 x span / 8 entries each.
-constexpr int fft_tw_offset(int P, int s) { return s == 0 ? 0 : fft_tw_offset(P, s - 1) + 3 * (P >> (3 * s)); }
-// Frequency of point p of the digit-reversed line.
-constexpr int fft_frequency(int P, int p)
-{
-    int f = 0, scale = 1, span = P;
-    for (int s = 0; s < fft_stages(P); ++s, scale *= 8, span /= 8) f += scale * (p / (span / 8) % 8);
-    return f + scale * (p % fft_mid(P));
-}
-
-__host__ __device__ constexpr int fft_swz(int i) { return i ^ ((i >> 3) & 31); }
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b)
 {
@@ -58,13 +21,18 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b)
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
 
-template <int N, class F> __device__ __forceinline__ void static_for(F &&f)
-{
-    if constexpr (N > 0) {
-        static_for<N - 1>(f);
-        f(std::integral_constant<int, N - 1>{});
-    }
-}
+// ---------------------------------------------------------------------------
+// Second LDS FFT: radix-8 Stockham passes (one radix-2 or radix-4 pass first
+// when log2 P is not a multiple of 3), so P = 8192 takes 5 passes instead of
+// 7.  The line is stored with one pad entry every 16 (index lpad(i)), which
+// spreads the strided writes of the early passes over all LDS banks.  The
+// twiddles come from an LDS copy of the first P/8 entries of the table
+// (w = exp(-+2 pi i base / P), base < P/8 in every radix-8 pass); the other
+// six powers of a butterfly are products of w (at most three multiplications
+// deep).  Length of the padded line: lds_len(P).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int lpad(int i) { return i + (i >> 4); }
+constexpr int lds_len(int P) { return P + P / 16; }
 
 template <bool INV>
 __device__ __forceinline__ void dft4(float2 &v0, float2 &v1, float2 &v2, float2 &v3)
@@ -110,184 +78,127 @@ __device__ __forceinline__ void dft_r(float2 (&v)[R])
     }
 }
 
-// a b, or a times the conjugate of b
-template <bool CONJ> __device__ __forceinline__ float2 cmul_or_conj(float2 a, float2 b)
+// Filter of the line: forward transform, product with the spectrum hs, inverse
+// transform.  load(j, v) gives butterfly j of the first pass its R inputs j + r
+// P/R, store(q, j, v) takes the results j + r P/8 of butterfly j of the last
+// pass, the thread's q-th: functors for all of a butterfly's points, so that
+// their memory accesses are in flight together, and no LDS round trip (and its
+// barriers) of their own.  The spectrum multiplies the last forward pass's
+// outputs.  after_load() runs between the inputs' loads and the first exchange,
+// before_store(q, j) ahead of the last pass.  STORE_LDS: store writes the LDS
+// line.
+template <int P, int NT, int R, int NS, bool INV, class Load, class AfterLoad, class Sync, class Put>
+__device__ __forceinline__ void fft_pass_io(const float2 *__restrict__ twl, Load load, AfterLoad after_load, Sync sync,
+                                            Put put)
 {
-    if (!CONJ) return cmul(a, b);
-    return make_float2(__builtin_fmaf(a.x, b.x, a.y * b.y), __builtin_fmaf(a.y, b.x, -a.x * b.y));
-}
-
-// v[m] w^m from the powers 1, 2 and 4 (CONJ: of the conjugate)
-template <bool CONJ> __device__ __forceinline__ void twiddle8(float2 (&v)[8], const float2 (&w)[3])
-{
-    const float2 w3 = cmul(w[0], w[1]);
-    v[1] = cmul_or_conj<CONJ>(v[1], w[0]);
-    v[2] = cmul_or_conj<CONJ>(v[2], w[1]);
-    v[3] = cmul_or_conj<CONJ>(v[3], w3);
-    v[4] = cmul_or_conj<CONJ>(v[4], w[2]);
-    v[5] = cmul_or_conj<CONJ>(v[5], cmul(w[0], w[2]));
-    v[6] = cmul_or_conj<CONJ>(v[6], cmul(w[1], w[2]));
-    v[7] = cmul_or_conj<CONJ>(v[7], cmul(w3, w[2]));
-}
-
-// the first stage's transform when points 4 .. 7 are zero
-__device__ __forceinline__ void dft8_half(float2 (&v)[8])
-{
-    constexpr float c = 0.70710678118654752440f;
-    float2 a[4] = {v[0], v[1], v[2], v[3]};
-    float2 b[4] = {v[0], make_float2(c * (v[1].x + v[1].y), c * (v[1].y - v[1].x)), make_float2(v[2].y, -v[2].x),
-                   make_float2(c * (v[3].y - v[3].x), -c * (v[3].x + v[3].y))};
-    dft4<false>(a[0], a[1], a[2], a[3]);
-    dft4<false>(b[0], b[1], b[2], b[3]);
+    constexpr int B = P / R, PER = (B + NT - 1) / NT, LR = ilog2c(R), L = ilog2c(P), LNS = ilog2c(NS);
+    const int t = threadIdx.x;
+    float2 v[PER][R];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        v[2 * m] = a[m];
-        v[2 * m + 1] = b[m];
+    for (int q = 0; q < PER; ++q) {
+        const int j = t + q * NT;
+        if (j < B) load(j, v[q]);
+    }
+    after_load();
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int j = t + q * NT;
+        if (j < B) {
+            if (R == 8 && NS > 1) {
+                const int k = j & (NS - 1);
+                float2 w1 = twl[k << (L - 3 - LNS)];
+                if (INV) w1.y = -w1.y;
+                const float2 w2 = cmul(w1, w1), w3 = cmul(w1, w2), w4 = cmul(w2, w2);
+                const float2 w5 = cmul(w1, w4), w6 = cmul(w3, w3), w7 = cmul(w3, w4);
+                const float2 w[8] = {make_float2(1.f, 0.f), w1, w2, w3, w4, w5, w6, w7};
+#pragma unroll
+                for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], w[r]);
+            }
+            dft_r<R, INV>(v[q]);
+        }
+    }
+    sync();
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int j = t + q * NT;
+        if (j < B) put(q, j, ((j >> LNS) << (LNS + LR)) + (j & (NS - 1)), v[q]);
     }
 }
 
-// Orders a stage's exchange among T consecutive threads.
-template <int T> __device__ __forceinline__ void fft_sync()
+// passes NS, 8 NS, ... up to but not including the last, LDS to LDS
+template <int P, int NT, int NS, bool INV>
+__device__ __forceinline__ void fft_mid_passes(float2 *a, const float2 *__restrict__ twl)
 {
-    if constexpr (T > 64) {
+    if constexpr (NS * 8 < P) {
+        auto load = [&](int j, float2 (&v)[8]) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) v[r] = a[lpad(j + r * (P / 8))];
+        };
+        auto put = [&](int, int, int d0, float2 (&v)[8]) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) a[lpad(d0 + r * NS)] = v[r];
+        };
+        fft_pass_io<P, NT, 8, NS, INV>(twl, load, [] {}, [] { __syncthreads(); }, put);
         __syncthreads();
-    } else {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        fft_mid_passes<P, NT, NS * 8, INV>(a, twl);
     }
 }
 
-// The eight points of butterfly j in the stage of stride T (span 8 T).
-template <int T> struct FftPoints {
-    int base;
-    __device__ __forceinline__ explicit FftPoints(int j) : base(fft_swz((j / T) * (8 * T) + (j & (T - 1)))) {}
-    // index bits of base and r T are disjoint, and fft_swz is linear in them
-    __device__ __forceinline__ int operator()(int r) const { return T >= 256 ? base + r * T : base ^ fft_swz(r * T); }
-};
-
-// Filter of the line.  load(j, v) gives inputs j + r P/8 in v[r], store(q, j, v)
-// takes those results (HALF: r < 4; the other inputs are zero and the other
-// results not wanted) of butterfly j, the thread's q-th; a functor for all of a
-// thread's points can have its loads in flight together.  after_load() runs
-// between the inputs' loads and the first exchange, before_store(q, j) ahead of
-// the last one.  tw: the stages' tables; hs: the spectrum in the order of
-// spectrum_order().
-template <int P, int NT, bool HALF, class Load, class AfterLoad, class BeforeStore, class Store>
+template <int P, int NT, bool STORE_LDS, class Load, class AfterLoad, class BeforeStore, class Store>
 __device__ __forceinline__ void fft_filter(float2 *a, const float2 *__restrict__ tw, const float *__restrict__ hs,
                                            Load load, AfterLoad after_load, BeforeStore before_store, Store store)
 {
-    constexpr int B = P / 8, PER = (B + NT - 1) / NT, S = fft_stages(P), R = fft_mid(P);
+    constexpr int L = ilog2c(P), FIRST = L % 3 == 1 ? 2 : (L % 3 == 2 ? 4 : 8), B = P / 8;   // FIRST: radix
+    constexpr int PER = (B + NT - 1) / NT;
+    static_assert(P > FIRST, "two passes or more");
     const int t = threadIdx.x;
-    // the twiddles of the next stage, requested ahead of its exchange
-    float2 w[PER][3];
-    auto fetch = [&](auto sc) {
-        constexpr int s = decltype(sc)::value, T = B >> (3 * s);
+    float2 *twl = a + lds_len(P);
+    for (int i = t; i < P / 8; i += NT) twl[i] = tw[i];   // read behind the first pass's barrier
+    auto nothing = [] {};
+    auto barrier = [] { __syncthreads(); };
+    auto from_lds = [&](int j, auto &v) {
+        constexpr int R = sizeof(v) / sizeof(float2);
 #pragma unroll
-        for (int q = 0; q < PER; ++q)
-#pragma unroll
-            for (int m = 0; m < 3; ++m) w[q][m] = tw[fft_tw_offset(P, s) + m * T + ((t + q * NT) & (T - 1))];
+        for (int r = 0; r < R; ++r) v[r] = a[lpad(j + r * (P / R))];
     };
-    fetch(std::integral_constant<int, 0>{});
-    float2 v[8];
+    auto first_put = [&](int, int, int d0, auto &v) {
+        constexpr int R = sizeof(v) / sizeof(float2);
 #pragma unroll
-    for (int q = 0; q < PER; ++q) {
-        const int j = t + q * NT;
-        if (j < B) {
-            load(j, v);
-            if constexpr (HALF) dft8_half(v);
-            else dft_r<8, false>(v);
-            twiddle8<false>(v, w[q]);
-            const FftPoints<B> at(j);
-#pragma unroll
-            for (int r = 0; r < 8; ++r) a[at(r)] = v[r];
-        }
-    }
-    after_load();
+        for (int r = 0; r < R; ++r) a[lpad(d0 + r)] = v[r];
+    };
+    fft_pass_io<P, NT, FIRST, 1, false>(twl, load, after_load, nothing, first_put);
+    __syncthreads();
+    fft_mid_passes<P, NT, FIRST, false>(a, twl);
+    // ahead of its use where the registers allow
+    constexpr bool AHEAD = P <= 4096;
     float h[PER][8];
-    auto next = [&](auto sc) {   // what follows forward stage s - 1
-        constexpr int s = decltype(sc)::value;
-        if constexpr (s < S) fetch(sc);
-        else
+    auto fetch = [&](int q, int j) {
 #pragma unroll
-            for (int q = 0; q < PER; ++q)
-#pragma unroll
-                for (int r = 0; r < 8; ++r) h[q][r] = hs[r * B + min(t + q * NT, B - 1)];
+        for (int r = 0; r < 8; ++r) h[q][r] = hs[j + r * B];
     };
-    next(std::integral_constant<int, 1>{});
-    fft_sync<B>();
-    static_for<S - 1>([&](auto sc) {
-        constexpr int s = decltype(sc)::value + 1, T = B >> (3 * s);
 #pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const int j = t + q * NT;
-            if (j < B) {
-                const FftPoints<T> at(j);
+    for (int q = 0; AHEAD && q < PER; ++q) fetch(q, min(t + q * NT, B - 1));
+    auto spectrum = [&](int q, int j, int, float2 (&v)[8]) {
+        if (!AHEAD) fetch(q, j);
 #pragma unroll
-                for (int r = 0; r < 8; ++r) v[r] = a[at(r)];
-                dft_r<8, false>(v);
-                twiddle8<false>(v, w[q]);
+        for (int r = 0; r < 8; ++r) a[lpad(j + r * B)] = make_float2(v[r].x * h[q][r], v[r].y * h[q][r]);
+    };
+    fft_pass_io<P, NT, 8, B, false>(twl, from_lds, nothing, barrier, spectrum);
+    __syncthreads();
+    fft_pass_io<P, NT, FIRST, 1, true>(twl, from_lds, nothing, barrier, first_put);
+    __syncthreads();
+    fft_mid_passes<P, NT, FIRST, true>(a, twl);
 #pragma unroll
-                for (int r = 0; r < 8; ++r) a[at(r)] = v[r];
-            }
-        }
-        next(std::integral_constant<int, s + 1>{});
-        fft_sync<T>();
-    });
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-        const int j = t + q * NT;
-        if (j < B) {
-            const FftPoints<1> at(j);
-#pragma unroll
-            for (int r = 0; r < 8; ++r) v[r] = a[at(r)];
-#pragma unroll
-            for (int g = 0; g < 8; g += R) {
-                float2 x[R];
-#pragma unroll
-                for (int r = 0; r < R; ++r) x[r] = v[g + r];
-                dft_r<R, false>(x);
-#pragma unroll
-                for (int r = 0; r < R; ++r) x[r] = make_float2(x[r].x * h[q][g + r], x[r].y * h[q][g + r]);
-                dft_r<R, true>(x);
-#pragma unroll
-                for (int r = 0; r < R; ++r) a[at(g + r)] = x[r];
-            }
-        }
-    }
-    static_for<S - 1>([&](auto sc) {
-        constexpr int s = S - 1 - decltype(sc)::value, T = B >> (3 * s);
-        fetch(std::integral_constant<int, s>{});
-        fft_sync<T>();
-#pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const int j = t + q * NT;
-            if (j < B) {
-                const FftPoints<T> at(j);
-#pragma unroll
-                for (int r = 0; r < 8; ++r) v[r] = a[at(r)];
-                twiddle8<true>(v, w[q]);
-                dft_r<8, true>(v);
-#pragma unroll
-                for (int r = 0; r < 8; ++r) a[at(r)] = v[r];
-            }
-        }
-    });
-    fetch(std::integral_constant<int, 0>{});
-#pragma unroll
-    for (int q = 0; q < PER; ++q) before_store(q, min(t + q * NT, B - 1));
-    fft_sync<B>();
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-        const int j = t + q * NT;
-        if (j < B) {
-            const FftPoints<B> at(j);
-#pragma unroll
-            for (int r = 0; r < 8; ++r) v[r] = a[at(r)];
-            twiddle8<true>(v, w[q]);
-            dft_r<8, true>(v);
-            store(q, j, v);
-        }
+    for (int q = 0; AHEAD && q < PER; ++q) before_store(q, min(t + q * NT, B - 1));
+    auto last = [&](int q, int j, int, float2 (&v)[8]) {
+        if (!AHEAD) before_store(q, j);
+        store(q, j, v);
+    };
+    if constexpr (STORE_LDS) {
+        fft_pass_io<P, NT, 8, B, true>(twl, from_lds, nothing, barrier, last);
+        __syncthreads();
+    } else {
+        fft_pass_io<P, NT, 8, B, true>(twl, from_lds, nothing, nothing, last);
     }
 }
 

@@ -37,8 +37,8 @@ struct RowFilterArgs {
                                 // mode 3
     int insert;                 // mode 0: nInsert; mode 1: (P - n) / 2
     const float *taper;         // mode 0: nInsert sigmoid weights
-    const float *hs;            // P real spectral multipliers (spectrum_order)
-    const float2 *tw;           // the stages' twiddles (make_twiddles)
+    const float *hs;            // P real spectral multipliers
+    const float2 *tw;           // P twiddles exp(-2 pi i k / P)
     float post0, post1, post2;  // sequential output multipliers
     const float *pre_w;         // mode 1: per-projection input weight (nullable)
     int rows_per_proj;          // rows of one projection (mode 1)
@@ -73,7 +73,6 @@ int filter_rows_to(mr_filter_plan *plan, const float *in, float *out, size_t n_r
 size_t filter_width(const mr_filter_plan *plan);
 int run_fdk_margin_rows(float *img, int n, int h, long n_proj, hipStream_t s);
 std::vector<float> make_twiddles(size_t P);
-std::vector<float> spectrum_order(const std::vector<float> &h);
 // Zero-fills n floats with a kernel (no hipMemset, so callers may capture it in a graph).
 int fill_zero(float *d, size_t n, hipStream_t s);
 

@@ -63,30 +63,25 @@ __device__ __forceinline__ float fdk_row_vv2(const RowFilterArgs &a, long r)
     return vv * vv;
 }
 
-// Threads of a block whose stages have NB butterflies (or more, at P = 16384):
-// one butterfly per thread; two at P = 8192, where the 1024 threads of a block
-// would have 64 registers each to keep two blocks on a CU and spill (20 000
-// rows of 4000: 308 us, 368 with one block of 1024 per CU, 515 with spills; at
-// P = 4096 two butterflies per thread take 542 us against 480).
-constexpr int filter_threads(int P, int NB) { return P == 8192 ? NB / 2 : NB; }
-
-// One row pair per block; dynamic LDS holds the line (P float2).  The padded
-// line is built in the first stage's loads and the kept samples are cropped and
-// scaled in the last stage: no LDS round trip of their own.  SHORT: modes 3 and
+// One row pair per block; dynamic LDS holds the padded line (lds_len(P) float2)
+// and the P/8 twiddles.  The padded line is built in the first pass's loads and
+// the kept samples are cropped and scaled in the last pass.  SHORT: modes 3 and
 // 4, whose rows (n <= P / 2 samples) fill the first half of the line.
 //
-// Bound by latency and issue together: at P = 4096 the vector ALU issues for
-// about half of the time and LDS is busy for a quarter (no bank conflicts), at
-// 8 waves per SIMD; hence all of a thread's global loads in flight at once, and
-// twiddles, spectrum and responses requested ahead of the exchange before their
-// use.  76 800 rows of 2048: 480 us (2.6 TB/s) against 676 with Stockham stages
-// (two block barriers each, the twiddles in LDS, 40 % of the LDS cycles bank
-// conflicts); with the normalisation of raw counts 625 against 885.
-template <int P, int NB, bool SHORT>
-__global__ __launch_bounds__(filter_threads(P, NB), P <= 4096 ? 8 : 4) void row_filter_kernel2(RowFilterArgs a)
+// Bound by VALU issue and latency together, so all of a butterfly's rows and
+// references are loaded before any is used (behind per-sample branches they came
+// one after the other), the rows' ends are normalised once per wave instead of
+// by every lane, spectrum and responses are requested a pass ahead, and the
+// passes are unrolled with constant strides.  Same values as before in every
+// bit.  76 800 rows of 2048: 676 -> 628 us, with the normalisation of raw counts
+// 885 -> 680; 20 000 of 4000 640 -> 541; 4000 of 8192 268 -> 221.  An in-place
+// transform (decimation in frequency, then in time: half the exchanges, no bank
+// conflicts) took 490 us for the first, but in filters that leave 1e-4 of a
+// row's norm its rounding differs from this order's by 3e-5 of the result.
+template <int P, int NT, bool SHORT>
+__global__ __launch_bounds__(NT, P <= 8192 ? 8 : 4) void row_filter_kernel2(RowFilterArgs a)
 {
     extern __shared__ float2 line[];
-    constexpr int NT = filter_threads(P, NB);
     const long r0 = 2 * (long)blockIdx.x;
     const bool has1 = r0 + 1 < a.n_rows;
     float *row0 = a.rows + r0 * a.n;
@@ -99,15 +94,16 @@ __global__ __launch_bounds__(filter_threads(P, NB), P <= 4096 ? 8 : 4) void row_
     auto nothing2 = [](int, int) {};
     // point by point: load(i) -> value, store(i, value)
     auto each = [](auto &load) {
-        return [&load](int j, float2 (&v)[8]) {
+        return [&load](int j, auto &v) {
+            constexpr int R = sizeof(v) / sizeof(float2);
 #pragma unroll
-            for (int r = 0; r < (SHORT ? 4 : 8); ++r) v[r] = load(j + r * B);
+            for (int r = 0; r < R; ++r) v[r] = load(j + r * (P / R));
         };
     };
     auto to_each = [](auto &store) {
         return [&store](int, int j, const float2 (&v)[8]) {
 #pragma unroll
-            for (int r = 0; r < (SHORT ? 4 : 8); ++r) store(j + r * B, v[r]);
+            for (int r = 0; r < 8; ++r) store(j + r * B, v[r]);
         };
     };
     if constexpr (SHORT) {
@@ -133,41 +129,45 @@ __global__ __launch_bounds__(filter_threads(P, NB), P <= 4096 ? 8 : 4) void row_
                 e = lognorm_value(e, flat, flat ? (second ? flat1 : flat0)[end] : 0.0f, dark,
                                   dark ? (second ? dark1 : dark0)[end] : 0.0f, second ? dl1 : dl0);
             const float f0 = __shfl(e, 0), l0 = __shfl(e, 1), f1 = __shfl(e, 2), l1 = __shfl(e, 3);
-            auto load = [&](int j, float2 (&v)[8]) {
-                int i[4];
-                float x0[4], x1[4], g0[4], g1[4], d0[4], d1[4];
+            // the upper half of the line is zero
+            auto load = [&](int j, auto &v) {
+                constexpr int R = sizeof(v) / sizeof(float2), H = R / 2, S = P / R;
+                int i[H];
+                float x0[H], x1[H], g0[H], g1[H], d0[H], d1[H];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    i[r] = min(j + r * B, a.n - 1);
+                for (int r = 0; r < H; ++r) {
+                    i[r] = min(j + r * S, a.n - 1);
                     x0[r] = row0[i[r]];
                     x1[r] = row1[i[r]];
                 }
                 if (norm) {
                     if (flat)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
+                        for (int r = 0; r < H; ++r) {
                             g0[r] = flat0[i[r]];
                             g1[r] = flat1[i[r]];
                         }
                     if (dark)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
+                        for (int r = 0; r < H; ++r) {
                             d0[r] = dark0[i[r]];
                             d1[r] = dark1[i[r]];
                         }
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
+                    for (int r = 0; r < H; ++r) {
                         x0[r] = lognorm_value(x0[r], flat, g0[r], dark, d0[r], dl0);
                         x1[r] = lognorm_value(x1[r], flat, g1[r], dark, d1[r], dl1);
                     }
                 }
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
+                for (int r = 0; r < H; ++r) {
                     const float s = (float)i[r] * a.ramp_inv, t1 = 1.0f - s;
-                    const bool in = j + r * B < a.n;
+                    const bool in = j + r * S < a.n;
                     v[r] = make_float2(in ? x0[r] - (f0 * t1 + l0 * s) : 0.0f,
                                        in && has1 ? x1[r] - (f1 * t1 + l1 * s) : 0.0f);
                 }
+#pragma unroll
+                for (int r = H; r < R; ++r) v[r] = make_float2(0.0f, 0.0f);
             };
             float rf[PER][4], rl[PER][4];
             auto before_store = [&](int q, int j) {
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(filter_threads(P, NB), P <= 4096 ? 8 : 4) void row_
                     }
                 }
             };
-            fft_filter<P, NT, true>(line, a.tw, a.hs, load, nothing, before_store, store);
+            fft_filter<P, NT, false>(line, a.tw, a.hs, load, nothing, before_store, store);
             return;
         }
         // mode 4: the rows' dot products with the responses fold back onto
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(filter_threads(P, NB), P <= 4096 ? 8 : 4) void row_
             o0[i] = y0;
             if (has1) o1[i] = y1;
         };
-        fft_filter<P, NT, true>(line, a.tw, a.hs, each(load), reduce, nothing2, to_each(store));
+        fft_filter<P, NT, false>(line, a.tw, a.hs, each(load), reduce, nothing2, to_each(store));
         return;
     } else if (a.mode == 0) {
         const float f0 = row0[0], l0 = row0[a.n - 1], f1 = row1[0], l1 = row1[a.n - 1];
@@ -275,9 +275,8 @@ __global__ __launch_bounds__(filter_threads(P, NB), P <= 4096 ? 8 : 4) void row_
             const bool in = d >= 0 && d < a.n;
             return make_float2(in ? row0[d] * a.post0 : 0.0f, (in && has1) ? row1[d] * a.post0 : 0.0f);
         };
-        auto store = [&](int i, float2 v) { line[fft_swz(i)] = v; };   // in place
-        fft_filter<P, NT, false>(line, a.tw, a.hs, each(load), nothing, nothing2, to_each(store));
-        __syncthreads();
+        auto store = [&](int i, float2 v) { line[lpad(i)] = v; };
+        fft_filter<P, NT, true>(line, a.tw, a.hs, each(load), nothing, nothing2, to_each(store));
         // adjoint of Pad: the tapers fold back onto the first and last sample
         // (left taper at 0..nInsert-1, right taper at P+15-j, inside the
         // FFT window only for j >= 16)
@@ -285,12 +284,12 @@ __global__ __launch_bounds__(filter_threads(P, NB), P <= 4096 ? 8 : 4) void row_
         float sl0 = 0.0f, sl1 = 0.0f, sr0 = 0.0f, sr1 = 0.0f;
         for (int j = t; j < a.insert; j += NT) {
             const float w = a.taper[j];
-            const float2 l = line[fft_swz(j)];
+            const float2 l = line[lpad(j)];
             sl0 += w * l.x;
             sl1 += w * l.y;
             const int jj = P + 15 - j;
             if (jj < P) {
-                const float2 r = line[fft_swz(jj)];
+                const float2 r = line[lpad(jj)];
                 sr0 += w * r.x;
                 sr1 += w * r.y;
             }
@@ -316,7 +315,7 @@ __global__ __launch_bounds__(filter_threads(P, NB), P <= 4096 ? 8 : 4) void row_
             R1 += red[wv][3];
         }
         for (int i = t; i < a.n; i += NT) {
-            const float2 v = line[fft_swz(i + a.insert)];
+            const float2 v = line[lpad(i + a.insert)];
             float y0 = v.x, y1 = v.y;
             if (i == 0) { y0 += L0; y1 += L1; }
             if (i == a.n - 1) { y0 += R0; y1 += R1; }
@@ -343,8 +342,15 @@ __global__ void fdk_margin_rows_kernel(float *img, int n, int h, long n_proj)
 template <int P>
 static int launch_row_filter(const RowFilterArgs &a, hipStream_t s)
 {
-    // butterflies of a stage, at least a wave
-    constexpr int NB = (P / 8) < 64 ? 64 : ((P / 8) > 1024 ? 1024 : (P / 8)), NT = filter_threads(P, NB);
+    // one radix-8 butterfly per thread and pass: P / 8 threads (at most
+    // 1024); measured for the 384 000 rows of 2048 at P = 8192: 6.75 ms with
+    // the padding, spectrum and crop fused into the first and last passes,
+    // 7.8-8.1 ms without, 9.3-9.8 ms with P / 16 threads, 19.75 ms with a
+    // radix-4 FFT; the line split into 4 or 8 wave-local FFTs of length P / 4
+    // or P / 8 (two block barriers per row pair instead of two per pass)
+    // took 11.0 / 8.4 ms (2 / 4 waves per SIMD); radix-16 passes with P / 16
+    // threads 6.52 against 6.49 ms
+    constexpr int NT2 = (P / 8) < 64 ? 64 : ((P / 8) > 1024 ? 1024 : (P / 8));
     const long pairs = (a.n_rows + 1) / 2;
     if (pairs == 0) return MR_OK;
     if (pairs > 0x7fffffffL) {
@@ -355,13 +361,13 @@ static int launch_row_filter(const RowFilterArgs &a, hipStream_t s)
                                                 : (a.mode == 1 ? "row_filter_fdk" : "row_filter_adjoint"),
                    s);
     MR_REQUIRE((a.mode != 3 && a.mode != 4) || (a.resp_first && a.resp_last), "short filter without responses");
-    constexpr size_t lds = sizeof(float2) * P;
+    constexpr size_t lds = sizeof(float2) * (lds_len(P) + P / 8);
     const bool shortf = a.mode == 3 || a.mode == 4;
     if (shortf) MR_REQUIRE(2 * (size_t)a.n <= P, "short filter longer than half its line");
-    const void *k = shortf ? (const void *)row_filter_kernel2<P, NB, true> : (const void *)row_filter_kernel2<P, NB, false>;
+    const void *k = shortf ? (const void *)row_filter_kernel2<P, NT2, true> : (const void *)row_filter_kernel2<P, NT2, false>;
     if (lds > 65536) MR_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    if (shortf) hipLaunchKernelGGL((row_filter_kernel2<P, NB, true>), dim3((unsigned)pairs), dim3(NT), lds, s, a);
-    else hipLaunchKernelGGL((row_filter_kernel2<P, NB, false>), dim3((unsigned)pairs), dim3(NT), lds, s, a);
+    if (shortf) hipLaunchKernelGGL((row_filter_kernel2<P, NT2, true>), dim3((unsigned)pairs), dim3(NT2), lds, s, a);
+    else hipLaunchKernelGGL((row_filter_kernel2<P, NT2, false>), dim3((unsigned)pairs), dim3(NT2), lds, s, a);
     MR_HIP(hipGetLastError());
     return MR_OK;
 }
@@ -394,33 +400,17 @@ int run_fdk_margin_rows(float *img, int n, int h, long n_proj, hipStream_t s)
     return MR_OK;
 }
 
-// The radix-8 stages' twiddles exp(-2 pi i m k / span), k < span / 8, for m = 1,
-// 2, 4 and spans P, P/8, ..., in double, rounded to float (P entries, the rest
-// zero).
+// P twiddles exp(-2 pi i k / P) in double, rounded to float.
 std::vector<float> make_twiddles(size_t P)
 {
-    std::vector<float> tw(2 * P, 0.0f);
+    std::vector<float> tw(2 * P);
     const double pi = 3.1415926535897932384626433832795;
-    for (int s = 0; s < fft_stages((int)P); ++s) {
-        const size_t span = P >> (3 * s), at = (size_t)fft_tw_offset((int)P, s);
-        for (size_t e = 0; e < 3 * span / 8; ++e) {
-            const size_t m = e / (span / 8), k = e % (span / 8);
-            const double ang = -2.0 * pi * (double)(k << m) / (double)span;
-            tw[2 * (at + e)] = (float)std::cos(ang);
-            tw[2 * (at + e) + 1] = (float)std::sin(ang);
-        }
+    for (size_t k = 0; k < P; ++k) {
+        const double ang = -2.0 * pi * (double)k / (double)P;
+        tw[2 * k] = (float)std::cos(ang);
+        tw[2 * k + 1] = (float)std::sin(ang);
     }
     return tw;
-}
-
-// A spectrum of P values in the order in which the middle stage's threads
-// read it: point 8 j + m of the digit-reversed line at m P/8 + j.
-std::vector<float> spectrum_order(const std::vector<float> &h)
-{
-    const int P = (int)h.size();
-    std::vector<float> o(h.size());
-    for (int p = 0; p < P; ++p) o[(size_t)(p % 8) * (P / 8) + p / 8] = h[fft_frequency(P, p)];
-    return o;
 }
 
 }  // namespace mr
@@ -577,9 +567,7 @@ extern "C" int mr_filter_plan_create(mr_filter_plan **plan, size_t width, int fi
     hipError_t e = hipMalloc(&p->d_hs, sizeof(float) * P);
     if (e == hipSuccess) e = hipMalloc(&p->d_taper, sizeof(float) * taper.size());
     if (e == hipSuccess) e = hipMalloc(&p->d_tw, sizeof(float2) * P);
-    // (P may exceed the kernels' lengths when the short form serves)
-    const std::vector<float> hso = mr::spectrum_order(hs);
-    if (e == hipSuccess) e = hipMemcpy(p->d_hs, hso.data(), sizeof(float) * P, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(p->d_hs, hs.data(), sizeof(float) * P, hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = hipMemcpy(p->d_taper, taper.data(), sizeof(float) * taper.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->d_tw, tw.data(), sizeof(float) * 2 * P, hipMemcpyHostToDevice);
@@ -589,12 +577,12 @@ extern "C" int mr_filter_plan_create(mr_filter_plan **plan, size_t width, int fi
                          ? mr::short_filter(P, width, n_insert, hs, taper, p->scale, hq, resp, resp_adj)
                          : 0;
     if (Q > 0) {
-        const std::vector<float> twq = mr::make_twiddles(Q), hqo = mr::spectrum_order(hq);
+        const std::vector<float> twq = mr::make_twiddles(Q);
         resp.insert(resp.end(), resp_adj.begin(), resp_adj.end());
         e = hipMalloc(&p->d_hq, sizeof(float) * Q);
         if (e == hipSuccess) e = hipMalloc(&p->d_twq, sizeof(float2) * Q);
         if (e == hipSuccess) e = hipMalloc(&p->d_resp, sizeof(float) * 4 * width);
-        if (e == hipSuccess) e = hipMemcpy(p->d_hq, hqo.data(), sizeof(float) * Q, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(p->d_hq, hq.data(), sizeof(float) * Q, hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(p->d_twq, twq.data(), sizeof(float) * 2 * Q, hipMemcpyHostToDevice);
         if (e == hipSuccess)
             e = hipMemcpy(p->d_resp, resp.data(), sizeof(float) * 4 * width, hipMemcpyHostToDevice);

@@ -1,5 +1,5 @@
-"""The in-place radix-8 filter line against a double-precision convolution of
-the same row with the same impulse response.
+"""The radix-8 filter line against a double-precision convolution of the same row
+with the same impulse response.
 
 Every line length from 64 to 16384 points, in the short form (the row fills at
 most half of the line) and as the full padded line, with odd row counts (the last
