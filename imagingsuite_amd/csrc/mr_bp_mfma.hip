@@ -584,20 +584,20 @@ int launch_bp_split_prep(const BpmArgs &a, const float *proj, const int *idx, co
     return MR_OK;
 }
 
-// Where the matrix-core form is the faster one (measured against
-// bp_lds_kernel, whole calls, fused): from 17 slices (two tiles of 16; 1024^2
-// x 32 x 625: 1.22 against 1.74 ms, 2048^2 x 256 x 300: 12.9 against 22.5; a
-// single tile leaves the weights' cost to 16 slices: 1024^2 x 16 x 500 0.77
-// against 0.75, 2048^2 x 5 x 1500 8.0 against 3.8) and from 1.5e9
-// voxel-projection updates, below which its extra launches cost what it saves
-// (512^2 x 32 x 360: 0.22 against 0.29 ms; 256^2 x 64 x 180: 0.11 against
-// 0.11).  Four projections must fit the 60 MiB chunk of the no-allocation
-// entry point, which gives the same bits by adding whole groups of four.
-// Tile: 32 x 32 voxels (half the staging per voxel, one block of 16 waves
-// per CU) for long scans over many tiles (1024^2 x 64 x 900: 2.83 against 3.01
-// ms, 2048^2 x 256 x 1500: 51 against 54), else 16 x 16 (four blocks per CU
-// overlap each other's ends; 774^2 x 170 x 126: 0.74 against 0.84 ms, 329^2 x
-// 51 x 1408: 0.79 against 1.03).
+// Where the matrix-core form is the faster one (whole calls, fused, against
+// bp_lds_kernel): from 17 slices, two tiles of 16 (1024^2 x 32 x 625: 1.40
+// against 1.71 ms, 2048^2 x 256 x 300: 13.3 against 20.0; a single tile leaves
+// the weights' cost to 16 slices: 1024^2 x 16 x 500 0.77 against 0.75) and from
+// 1.5e9 voxel-projection updates, below which its extra launches cost what it
+// saves (300^2 x 40 x 450, 1.6e9: 0.25 against 0.24 ms; 400^2 x 40 x 300, 1.9e9:
+// 0.20 against 0.26; 512^2 x 32 x 360: 0.23 against 0.27).  Four projections must
+// fit the 60 MiB chunk of the no-allocation entry point, which gives the same
+// bits by adding whole groups of four.
+// Tile: 32 x 32 voxels (half the staging per voxel, one block of 16 waves per
+// CU) for long scans over many tiles (2048^2 x 256 x 1500: 62.9 against 68.0 ms,
+// 1024^2 x 64 x 900: 3.01 against 3.11), else 16 x 16 (four blocks per CU overlap
+// each other's ends; 774^2 x 170 x 126: 0.82 against 0.88 ms, 329^2 x 51 x 1408:
+// 0.83 against 1.06; 1024^2 x 64 x 300: 1.04 either way).
 bool bpm_shape(int nu, int nv, int nk, int &tile)
 {
     const size_t proj_bytes = 8 * (size_t)bpm_npair(nu) * (size_t)bpm_vp(nv);

@@ -155,8 +155,9 @@ class BackProjector:
     (ROI-relative), ``direction`` 0 = CW, 1 = CCW, ``buffer_size`` is
     ProjectionBufferSize (16 reproduces the reference exactly, including its
     dropped projections; 0 back-projects every projection).  ``fused`` folds
-    the interpolation into fused multiply-adds (float rounding differs from
-    the reference; otherwise results are bit-identical).
+    the interpolation into fused multiply-adds or, for large stacks, runs it on
+    the matrix cores in split halves (float rounding differs from the
+    reference; otherwise results are bit-identical).
 
     ``correct_tilt`` runs the module's bCorrectTilt branch with
     ``tilt_angle`` (degrees) and ``tilt_pivot`` (detector row); ``row0`` is
@@ -445,8 +446,7 @@ class BatchReconstructor:
     (mr_batch_*).  ``stacks`` is a list of dicts with keys proj (CUDA
     [n_proj, slices, width]), angles, weights, center and optionally
     filtertype, cutoff, direction, buffer_size; volumes are allocated here.
-    ``fused`` folds the interpolation into FMAs (float rounding only);
-    otherwise every stack is bit-identical to MultiProjBPparallel."""
+    ``fused`` as BackProjector's (float rounding only); otherwise every stack is bit-identical to MultiProjBPparallel."""
 
     def __init__(self, stacks, tune: bool = True, fused: bool = False):
         import torch

@@ -80,8 +80,8 @@ int mr_filter_plan_info(const mr_filter_plan *plan, size_t *fft_size, size_t *n_
 /* The kernel form this plan launches, e.g. "row_filter_kernel2<4096,512> short"
  * (the filter as a 4096-point convolution plus the taper responses, when
  * 2 width - 1 fits a power of two below the FFT length) or
- * "row_filter_kernel2<8192,1024>".  Diagnostics only; no counterpart in the
- * reference. */
+ * "row_filter_kernel2<8192,1024>": points, butterflies of a stage (at most
+ * 1024).  Diagnostics only; no counterpart in the reference. */
 int mr_filter_plan_kernel(const mr_filter_plan *plan, char *name, size_t len);
 /* Filters n_rows rows of `width` samples in place (device memory).  A projection
  * stack [n_proj][rows][width] is n_proj*rows rows. */
@@ -114,8 +114,10 @@ typedef struct {
     int use_roi;         /* MatrixInfo.bUseROI */
     size_t roi[4];       /* MatrixInfo.roi x0,y0,x1,y1 (inclusive) */
     int fused;           /* 0: the reference's float operation order per voxel (bit-identical
-                            results); 1: interpolation folded into fused multiply-adds
-                            (differs by float rounding only) */
+                            results); 1: float rounding only: interpolation folded into
+                            fused multiply-adds, or for large stacks (17 slices or more,
+                            see mr_bp_plan_kernel) on the matrix cores with every factor
+                            split into two halves, at least as near to double */
     /* Axis-tilt correction, the bCorrectTilt branches of the three back-projectors
      * (MultiProjBPparallel.cpp:49-114, MultiProjBP.cpp:50-96, NNMultiProjBP.cpp:48-81)
      * and the mask shrink of BuildCircleMask (BackProjectorModuleBase.cpp:171-180).
@@ -137,8 +139,10 @@ int mr_bp_plan_create(mr_bp_plan **plan, const mr_bp_params *params);
 int mr_bp_plan_destroy(mr_bp_plan *plan);
 /* Name of the kernel variant mr_bp_parallel launches for this plan (slice
  * tile, projection chunk, block order), e.g.
- * "bp_lds_kernel<32,0,false,4> order=1 sw=4".  Diagnostics only; no
- * counterpart in the reference. */
+ * "bp_lds_kernel<32,0,false,4,1> order=1 sw=4".  Once the plan has projected,
+ * the variant that its number of projections selects: also
+ * "bp_mfma_kernel tile=32" (fused plans) and the thin tiles of small grids.
+ * Diagnostics only; no counterpart in the reference. */
 int mr_bp_plan_kernel(const mr_bp_plan *plan, char *name, size_t len);
 /* Host copy of the circle mask: for row y the voxels first[y] <= x < second[y]
  * are reconstructed (BuildCircleMask's pair, with `second` exclusive). */
@@ -374,8 +378,9 @@ typedef struct mr_batch_plan mr_batch_plan;
 
 /* flags: MR_BATCH_TUNE - the autotuner times every (slice tile, projection
  * chunk) variant of the persistent kernel on this batch and keeps the
- * fastest; MR_BATCH_FUSED - the interpolation is folded into two FMAs per
- * update (as mr_bp_params.fused; float rounding only), otherwise every stack
+ * fastest; MR_BATCH_FUSED - as mr_bp_params.fused (float rounding only; the
+ * larger stacks run on the matrix cores, which mr_batch_plan_info reports as
+ * slice tile 64 when all do), otherwise every stack
  * keeps MultiProjBPparallel's operation order.  Unknown bits: MR_ERR_INVALID. */
 #define MR_BATCH_TUNE 1
 #define MR_BATCH_FUSED 2
