@@ -705,8 +705,8 @@ static int launch_bp(const BpArgs &a, hipStream_t s)
 // read when needed and one window position after the other: 1024^2 x 64 x 900
 // 8.4 against 7.1 ms, 512^2 x 16 x 360 0.63 against 0.50, 256^2 x 36 x 180 -
 // then nine 4-slice tiles instead of three of 16 - 0.44 against 0.23.)  Bound
-// by the LDS reads of the windows (about 55 % of the cycles before, 65 % now)
-// and the latency of a line.
+// by the LDS reads of the windows (55 % of the cycles) and the latency of a line
+// (43 % of the wave cycles wait).
 //
 // On one line the detector position u is monotone along the line with slope
 // |sin| (or |cos|) >= 1/sqrt 2, so the voxels a bin receives from form one
