@@ -202,8 +202,8 @@ __global__ __launch_bounds__(256) void fdk_kernel(FdkArgs a)
 // each (plain vector-register float operations issue at 2.4 if another wave's
 // can be paired, operations with a scalar operand, conversions and shifts at
 // 4.4, DPP at 4.4 unpaired), 26 cycles in all at 2.0 GHz; staging takes 15 of
-// the 114 ms below.  Where fdk_kernel's gathers keep the texture addresser busy
-// at 16 cycles each.  1024^3 x 720: 114 + 2 (transposition) against 149 ms,
+// the 114 ms below.  (fdk_kernel's gathers take the texture addresser 16 cycles
+// each.)  1024^3 x 720: 114 + 2 (transposition) against 149 ms,
 // fused 92 + 2 against 134; 512^2 x 256 x 400: 4.5 + 0.2 against 5.3.  Blocks
 // of 2 waves (8 x 4 columns): 146, of 8 waves (8 x 16): 119 ms.
 // ---------------------------------------------------------------------------

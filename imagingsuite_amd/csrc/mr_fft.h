@@ -1,10 +1,9 @@
 // LDS-resident Stockham FFT for one complex line of compile-time length P,
 // shared by the parallel-beam and the FDK ramp filters.
 //
-// The line lives in LDS as float2[P].  Passes are radix-4 (plus one radix-2
-// pass first when log2 P is odd); every pass reads its butterfly inputs into
-// registers, synchronises, and writes the outputs back in natural (Stockham
-// autosort) order, so no bit reversal is needed.  Twiddles come from a
+// The line lives in LDS as float2, padded (lpad); every pass reads its butterfly
+// inputs into registers, synchronises, and writes the outputs back in natural
+// (Stockham autosort) order, so no bit reversal is needed.  Twiddles come from a
 // P-entry table tw[k] = exp(-2 pi i k / P) computed in double on the host.
 #pragma once
 
@@ -22,7 +21,7 @@ __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
 
 // ---------------------------------------------------------------------------
-// Second LDS FFT: radix-8 Stockham passes (one radix-2 or radix-4 pass first
+// Radix-8 Stockham passes (one radix-2 or radix-4 pass first
 // when log2 P is not a multiple of 3), so P = 8192 takes 5 passes instead of
 // 7.  The line is stored with one pad entry every 16 (index lpad(i)), which
 // spreads the strided writes of the early passes over all LDS banks.  The
