@@ -363,7 +363,7 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
         inside = x >= m.x && x < m.y;
     }
     const bool any_inside = __syncthreads_or(inside ? 1 : 0) != 0;
-    if (any_inside && zl > 0) {
+    if (any_inside && zl > 0 && a.nk > 0) {   // (no projection: the table has no entry to read)
         const float yf = (float)(y + 1), xf = (float)(x + 1);
         const int num2 = a.nu - 2;
         // Staging: wave w takes projections w, w + 4, ... of a chunk, each as
