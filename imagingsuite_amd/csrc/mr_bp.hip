@@ -429,7 +429,7 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
         };
         int low = lowest(0), low_next = low;
         stage(0, low, lds.buf[0]);
-        __syncthreads();
+        lds_loads_barrier();
         for (int kb = 0, buf = 0; kb < a.nk; kb += C, buf ^= 1) {
             const int kc = min(C, a.nk - kb);
             const float (&sm)[C][SPAN][RS] = lds.buf[buf];
@@ -578,7 +578,7 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
             }
             }
             low = low_next;
-            __syncthreads();
+            lds_loads_barrier();
         }
     }
     if (!in_vol) return;
@@ -934,7 +934,7 @@ __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict
         nxt[r] = uniform(spans[R + r]);
     }
     stage(1 + sr, uniform(spans[sr]), 0);
-    __syncthreads();
+    lds_loads_barrier();
     for (int L = 1, buf = 0; L <= nu; L += R, buf ^= 1) {
         int2 far[R], mine = nxt[0];
 #pragma unroll
@@ -954,7 +954,7 @@ __global__ __launch_bounds__(256) void bp_adjoint_kernel(const float *__restrict
             cur[r] = nxt[r];
             nxt[r] = uniform(far[r]);
         }
-        __syncthreads();
+        lds_loads_barrier();
     }
     // bins 1 and nu - 1 of the linear form are bp_adjoint_edge_kernel's
     if (!active || (INTERP == 0 && (u == 1 || u == nu - 1))) return;

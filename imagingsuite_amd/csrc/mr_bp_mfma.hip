@@ -466,7 +466,7 @@ __device__ __forceinline__ void bpm_tile(const BpmArgs &a, int bx, int by, int b
         bool edge = !__all(lo >= 0.0f && hi < fnu1);
         stage(0, s0, lds);
         stage_table(4, 1);
-        __syncthreads();
+        lds_loads_barrier();
         int buf = 0;
         for (int kb = 0; kb < a.nk; kb += 4) {
             const int slot = (kb >> 2) & 1;
@@ -481,13 +481,13 @@ __device__ __forceinline__ void bpm_tile(const BpmArgs &a, int bx, int by, int b
             }
             update(cur, t, s0, edge);
             if (NB == 1) {
-                __syncthreads();
+                lds_loads_barrier();
                 if (kb + 4 < a.nk) stage(kb + 4, s1, lds);
             }
             t = valid(ltab[4 * (slot ^ 1) + g], kb + 4);   // read again: registers are short in update
             s0 = s1;
             edge = edge1;
-            __syncthreads();
+            lds_loads_barrier();
         }
     }
     float inv[NT];

@@ -44,6 +44,16 @@ __device__ __forceinline__ float4 tab_entry(const float4 *tab, int i)
 #endif
 }
 
+// Barrier of kernels that load straight into LDS: a wave's loads have arrived
+// once its vector-memory counter is zero, and the other waves may read them
+// once every wave has waited for that and passed the barrier.  __syncthreads()
+// does not promise the wait (the compiler of ROCm 7.2 happens to put it there).
+__device__ __forceinline__ void lds_loads_barrier()
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
 }  // namespace mr
 
 #define MR_HIP(call)                                                              \

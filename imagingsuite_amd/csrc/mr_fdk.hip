@@ -380,7 +380,7 @@ __global__ __launch_bounds__(kFsThreads, 4) void fdk_slice_kernel(FdkSliceArgs a
             // would wait for the direct loads behind them
 #pragma unroll
             for (int g = 0; g < GZ; ++g) asm volatile("" : "+v"(zt[g]));
-            __syncthreads();
+            lds_loads_barrier();
             for (int p = 0; p < a.np; ++p) {
                 float *cur = fs_lds + (p & 1) * a.bufw;
                 int r1 = 0, c1 = 0;
@@ -458,7 +458,7 @@ __global__ __launch_bounds__(kFsThreads, 4) void fdk_slice_kernel(FdkSliceArgs a
                     zt[g] = zn[g];
                     asm volatile("" : "+v"(zt[g]));
                 }
-                __syncthreads();
+                lds_loads_barrier();
             }
         };
         bool low = false;

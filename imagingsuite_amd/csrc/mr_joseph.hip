@@ -382,7 +382,7 @@ __global__ __launch_bounds__(256, R == 4 ? 4 : 5) void joseph_forward_dma_kernel
         nxt[r] = span(R + r);
     }
     stage(sr, span(sr), seg[0][sr]);
-    __syncthreads();
+    lds_loads_barrier();
     for (int L0 = 0, buf = 0; L0 < N; L0 += R, buf ^= 1) {
         int2 far[R];
 #pragma unroll
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(256, R == 4 ? 4 : 5) void joseph_forward_dma_kernel
             cur[r] = nxt[r];
             nxt[r] = make_int2(__builtin_amdgcn_readfirstlane(far[r].x), __builtin_amdgcn_readfirstlane(far[r].y));
         }
-        __syncthreads();
+        lds_loads_barrier();
     }
     if (!active) return;
     float *out = a.dst + ((size_t)ang * a.nd + n) * a.nz + z0;
@@ -547,7 +547,7 @@ __global__ __launch_bounds__(256) void joseph_adjoint_lds_kernel(JosephArgs a, i
     };
     int low = lowest(0), low_next = low;
     stage(0, low, sm[0]);
-    __syncthreads();
+    lds_loads_barrier();
     for (int kb = 0, buf = 0; kb < a.na; kb += C, buf ^= 1) {
         if (kb + C < a.na) {
             if (((kb + C) & 63) == 0) low_next = lowest(kb + C);
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(256) void joseph_adjoint_lds_kernel(JosephArgs a, i
             }
         }
         low = low_next;
-        __syncthreads();
+        lds_loads_barrier();
     }
     if (!in_vol) return;
     float *out = a.dst + ((size_t)y * N + x) * a.nz + z0;
