@@ -332,13 +332,6 @@ constexpr int kBpSpan = 26;
 // as in bp_tilt_kernel (1 MultiProjBPparallel, 2 MultiProjBP, 3
 // NearestNeighborBP): the detector position shifted by centeroffset and the
 // interpolation weight recomputed per slice group.
-// Whether the slices past the last group of four belong to the last tile that
-// has one.  Tiles of their own, all at the end of the tile list, leave the XCDs
-// that get them idle (1024^2 x 33 x 250: 1.43 against 0.82 ms); the 8-slice tilt
-// tiles keep them (the other registers that the two lines more give them cost 3
-// to 10 % at 8 to 15 slices).
-constexpr bool bp_last_tile_ends(int zt, int tilt) { return zt != 8 || tilt == 0; }
-
 template <int ZT, int KC> struct BpStage {
     static constexpr int C = ZT == 32 || KC <= 4 ? KC : KC / 2;
     float buf[2][C][kBpSpan][ZT + 4];
@@ -370,7 +363,7 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
         inside = x >= m.x && x < m.y;
     }
     const bool any_inside = __syncthreads_or(inside ? 1 : 0) != 0;
-    if (any_inside && zl > 0 && a.nk > 0) {   // (no projection: the table has no entry to read)
+    if (any_inside && zl > 0) {
         const float yf = (float)(y + 1), xf = (float)(x + 1);
         const int num2 = a.nu - 2;
         // Staging: wave w takes projections w, w + 4, ... of a chunk, each as
@@ -392,8 +385,11 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
         }
         // lowest column of projection 64 j + lane: one bin of margin, an interior
         // voxel may round one ulp below a corner and truncate to the bin below
+        // (the table has an entry 0 also when no projection is used; a branch
+        // around all this for that case costs up to 8 %, as the loop then compiles
+        // to other code)
         auto lowest = [&](int kb) {
-            const float4 t = a.tab[min(kb + lane, a.nk - 1)];
+            const float4 t = a.tab[max(min(kb + lane, a.nk - 1), 0)];
             const float ya = (float)(y0 + 1), yb = (float)(y0 + T);
             const float xa = (float)(x0 + 1), xb = (float)(x0 + T);
             int n0;
@@ -621,17 +617,16 @@ __device__ __forceinline__ void bp_lds_tile(const BpArgs &a, int bx, int by, int
         for (int g = 0; g < G; ++g)
             *reinterpret_cast<float4 *>(out + 4 * g) =
                 make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
-        return;
-    }
-    if constexpr (ZT < 16) {
+    } else if constexpr (ZT < 16) {
 #pragma unroll
         for (int z = 0; z < ZT; ++z)
             if (z < zn) out[z] = acc[z];
+        // slices past the one group of four: written here, where they share the
+        // lines (2048^2 x 7 x 48: 0.17 against 0.19 ms by bp_tail_kernel)
+        if constexpr (ZT == 4)
+            if (a.nz4 == 4 && !a.accumulate)
+                for (int z = 4; z < a.nv; ++z) out[z] = 0.0f;
     }
-    if constexpr (bp_last_tile_ends(ZT, TILT))
-        if (z0 + ZT >= a.nz4 && !a.accumulate)
-#pragma unroll 1
-            for (int z = ZT; z0 + z < a.nv; ++z) out[z] = 0.0f;
 }
 
 template <int ZT, int INTERP, bool EXACT, int KC, int PIPE>
@@ -1097,10 +1092,10 @@ __global__ __launch_bounds__(64) void bp_adjoint_edge_kernel(const float *__rest
 // Grid of the tiled kernel (16 x 16 voxel tiles): the XCD-striped 1-D grid
 // with stripes of 4 tile columns (order 1, see tile_of_block), or the 3-D
 // tile grid when the tile count would overflow the int tile numbers.
-static dim3 tiled_grid(BpArgs &a, int ZT, int tilt)
+static dim3 tiled_grid(BpArgs &a, int ZT)
 {
     a.ntx = a.nty = (a.nu + 15) / 16;
-    a.ntz = ((bp_last_tile_ends(ZT, tilt) ? std::max(1, a.nz4) : a.nv) + ZT - 1) / ZT;
+    a.ntz = (std::max(1, a.nz4) + ZT - 1) / ZT;
     const long n = (long)a.ntx * a.nty * a.ntz;
     a.order = n < (1L << 30) ? 1 : 0;
     a.sw = 4;
@@ -1108,27 +1103,52 @@ static dim3 tiled_grid(BpArgs &a, int ZT, int tilt)
     return dim3((unsigned)(8 * ((n + 7) / 8)));
 }
 
+// Zeroes the slices past the last group of four where that group ends a tile of
+// ZT slices.  Tiles of their own, all at the end of the tile list, would leave the
+// XCDs that get them idle (1024^2 x 33 x 250: 1.43 against 0.82 ms); as a few lines
+// more in the tiles they cost up to 8 % at 8 slices per tile.
+__global__ __launch_bounds__(256) void bp_tail_kernel(BpArgs a)
+{
+    if (a.gate && *a.gate == 0) return;
+    const int rest = a.nv - a.nz4;   // 1, 2 or 3
+    const size_t n = (size_t)a.nu * a.nu * rest;
+    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) {
+        const size_t v = e / rest;
+        a.vol[v * a.nv + a.nz4 + (e - v * rest)] = 0.0f;
+    }
+}
+
+static int launch_bp_tail(const BpArgs &a, int ZT, hipStream_t s)
+{
+    // (one group of four: the 4-slice tiles of every kernel write the rest)
+    if (a.accumulate || a.nz4 <= 4 || a.nz4 % ZT != 0 || a.nv == a.nz4) return MR_OK;
+    const size_t n = (size_t)a.nu * a.nu * (a.nv - a.nz4);
+    hipLaunchKernelGGL(bp_tail_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 16384)), dim3(256), 0, s, a);
+    MR_HIP(hipGetLastError());
+    return MR_OK;
+}
+
 template <int ZT, int INTERP, bool EXACT, int KC, int PIPE>
 static int launch_bp_lds(BpArgs a, hipStream_t s)
 {
-    const dim3 grid = tiled_grid(a, ZT, 0);
+    const dim3 grid = tiled_grid(a, ZT);
     ProfScope prof("bp_parallel", s);
     hipLaunchKernelGGL((bp_lds_kernel<ZT, INTERP, EXACT, KC, PIPE>), grid, dim3(256), 0, s, a);
     MR_HIP(hipGetLastError());
-    return MR_OK;
+    return launch_bp_tail(a, ZT, s);
 }
 
 // Tilt branches on the LDS-staged tiles (the reference order, rolled loop).
 template <int ZT, int KC>
 static int launch_bp_lds_tilt(BpArgs a, hipStream_t s)
 {
-    const dim3 grid = tiled_grid(a, ZT, a.tilt);
+    const dim3 grid = tiled_grid(a, ZT);
     ProfScope prof("bp_parallel_tilt", s);
     if (a.tilt == 1) hipLaunchKernelGGL((bp_lds_tilt_kernel<ZT, 0, KC, 1>), grid, dim3(256), 0, s, a);
     else if (a.tilt == 2) hipLaunchKernelGGL((bp_lds_tilt_kernel<ZT, 0, KC, 2>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((bp_lds_tilt_kernel<ZT, 1, KC, 3>), grid, dim3(256), 0, s, a);
     MR_HIP(hipGetLastError());
-    return MR_OK;
+    return launch_bp_tail(a, ZT, s);
 }
 
 template <int ZT, int KC, int PIPE>

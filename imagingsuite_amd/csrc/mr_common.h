@@ -50,7 +50,9 @@ __device__ __forceinline__ float4 tab_entry(const float4 *tab, int i)
 // does not promise the wait (the compiler of ROCm 7.2 happens to put it there).
 __device__ __forceinline__ void lds_loads_barrier()
 {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt 0, no wait on the other counters
+#endif
     __syncthreads();
 }
 
