@@ -1187,15 +1187,15 @@ static void lds_shape_tilt(int nu, int nv, int &zt, int &kc)
 // latencies of a block's chunks nor issue at full rate (one wave: 8 cycles per
 // instruction, four: 2.4), so a grid of few blocks takes thinner slice tiles,
 // unrolled and with chunks of 16: 4 slices where 8 would make at most one block
-// per CU, else 8 where the shape above has fewer than 4 blocks per CU or fewer
+// per CU, else 8 where the shape above has fewer than 800 blocks or fewer
 // than 16 slices (not below 8 slices: the unrolled tile would add zeros).  The
 // positions and weights, computed once per tile, are then computed more often.
 // Exact, in microseconds (shape above, 4, 8 slices): 128^2 x 16 x 180: 81, 38,
 // 46; 256^2 x 8 x 180: 58, 38, 47; 256^2 x 16 x 180: 67, 53, 49; 400^2 x 16 x
 // 360: 143, 168, 130; 300^2 x 10 x 700: 222, 190, 183; 512^2 x 8 x 360: 129,
-// 160, 113; 512^2 x 16 x 360 (1024 blocks): 190, -, 206; 1024^2 x 4 x 200: 156,
-// 153, 187.  Fewer than 32 projections are two chunks whichever way and keep
-// the shape above.
+// 160, 113; 440^2 x 16 x 250 (784 blocks): 143, -, 126; 450^2 x 16 x 250 (841): 143,
+// -, 153; 512^2 x 16 x 360 (1024): 190, -, 206; 1024^2 x 4 x 200: 156, 153, 187.
+// Fewer than 32 projections are two chunks whichever way and keep the shape above.
 static void lds_shape_nk(int nu, int nv, int nk, int &zt, int &kc, int &pipe)
 {
     lds_shape(nu, nv, zt, kc, pipe);
@@ -1205,7 +1205,7 @@ static void lds_shape_nk(int nu, int nv, int nk, int &zt, int &kc, int &pipe)
         zt = 4;
         kc = 16;
         pipe = 1;
-    } else if (nv >= 8 && (zt == 8 || tiles * ((nv + 15) / 16) < 1024)) {
+    } else if (nv >= 8 && (zt == 8 || tiles * (((nv & ~3) + 15) / 16) < 800)) {
         zt = 8;
         kc = 16;
         pipe = 1;
