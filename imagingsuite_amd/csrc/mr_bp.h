@@ -57,14 +57,14 @@ struct BpmArgs {
     const int2 *mask;
     const float2 *scale;     // per slice: factor on the samples, its inverse
     const int *flag;         // set: the samples do not fit the split, the kernel leaves at once
-    int nu, nv, vp, npair, nk, nz4;   // vp: slices rounded up to 16; npair: column pairs
+    int nu, nv, vp, npair, nk, nz4;   // vp: slices of whole groups of four, rounded up to 16; npair: column pairs
     int chain;               // 1: the volume holds the sums of earlier projections, continue them
     int ntx, nty, ntz, zt0, sw;
 };
 // Voxel tile of the matrix-core kernel for a stack with nk used projections,
 // or false where the VALU kernel serves it.
 bool bpm_shape(int nu, int nv, int nk, int &tile);
-inline int bpm_vp(int nv) { return (nv + 15) & ~15; }
+inline int bpm_vp(int nv) { return ((nv & ~3) + 15) & ~15; }
 inline int bpm_npair(int nu) { return (nu + 1) / 2; }
 size_t bpm_part_words(size_t nv, size_t nk);   // words of launch_bp_scale's partial maxima
 int launch_bp_scale(const float *proj, const int *idx, const float *wts, int nu, int nv, int nk, unsigned *part,

@@ -507,6 +507,8 @@ __device__ __forceinline__ void bpm_tile(const BpmArgs &a, int bx, int by, int b
 #pragma unroll
             for (int zt = 0; zt < NT; ++zt)
                 if (z0 + 16 * zt + m < a.nv) out[16 * zt] = in ? acc[q][zt][i] * inv[zt] : 0.0f;
+            // up to three slices past the last group of four, where that ends a tile
+            if (z0 + 16 * NT == a.nz4 && a.nz4 + m < a.nv) out[16 * NT] = 0.0f;
         }
     }
 }
@@ -577,7 +579,8 @@ int launch_bp_split_prep(const BpmArgs &a, const float *proj, const int *idx, co
                          hipStream_t s)
 {
     ProfScope prof("bp_prep", s);
-    dim3 g((unsigned)((2 * a.npair + 63) / 64), (unsigned)((a.vp + 63) / 64), (unsigned)a.nk);
+    // (vpad, the float sinogram's slices, exceeds vp where nv % 16 is 1, 2 or 3)
+    dim3 g((unsigned)((2 * a.npair + 63) / 64), (unsigned)((std::max(a.vp, vpad) + 63) / 64), (unsigned)a.nk);
     hipLaunchKernelGGL(bp_split_prep_kernel, g, dim3(256), 0, s, proj, const_cast<unsigned *>(a.split), idx, wts,
                        a.scale, a.flag, a.nu, a.nv, a.nz4, vpad, a.vp, a.npair);
     MR_HIP(hipGetLastError());
@@ -585,14 +588,21 @@ int launch_bp_split_prep(const BpmArgs &a, const float *proj, const int *idx, co
 }
 
 // Where the matrix-core form is the faster one (whole calls, fused, against
-// bp_lds_kernel): from 17 slices, two tiles of 16 (1024^2 x 32 x 625: 1.40
-// against 1.71 ms, 2048^2 x 256 x 300: 13.3 against 20.0; a single tile leaves
-// the weights' cost to 16 slices: 1024^2 x 16 x 500 0.77 against 0.75) and from
-// 1.5e9 voxel-projection updates, below which its extra launches cost what it
-// saves (300^2 x 40 x 450, 1.6e9: 0.25 against 0.24 ms; 400^2 x 40 x 300, 1.9e9:
-// 0.20 against 0.26; 512^2 x 32 x 360: 0.23 against 0.27).  Four projections must
-// fit the 60 MiB chunk of the no-allocation entry point, which gives the same
-// bits by adding whole groups of four.
+// bp_lds_kernel): from 17 slices (1024^2 x 32 x 625: 1.40 against 1.71 ms, 2048^2 x
+// 256 x 300: 13.3 against 20.0; a single tile of 16 leaves the weights' cost to 16
+// slices: equal from 400^2) and from 1.5e9 voxel-projection updates, below which
+// its extra launches cost what it saves (300^2 x 40 x 450, 1.6e9: 0.25 against 0.24
+// ms; 400^2 x 40 x 300, 1.9e9: 0.20 against 0.26; 512^2 x 32 x 360: 0.23 against
+// 0.27).  Each of its one or two launches (run_bpm: chunks of four slice tiles, then
+// a chunk of the rest) must have about two blocks per CU, as a block's own latency
+// is long: with 484 blocks 350^2 x 64 x 511 0.32 against 0.40 ms, 350^2 x 80 x 409
+// 0.39 against 0.50; with 361 300^2 x 64 x 382 0.24 either way, 300^2 x 100 x 445
+// equal; with 256 256^2 x 80 x 763 0.62 against 0.40 and with 64 128^2 x 100 x 916
+// 0.84 against 0.35.  One or two slice tiles need as much work per column of
+// blocks (350^2 x 32 x 1021: 0.41 against 0.50, 400^2 x 20 x 1250 0.55 against 0.57,
+// but 350^2 x 24 x 511 0.22 against 0.20, 300^2 x 32 x 1046 even).  Four
+// projections must fit the 60 MiB chunk of the no-allocation entry point, which
+// gives the same bits by adding whole groups of four.
 // Tile: 32 x 32 voxels (half the staging per voxel, one block of 16 waves per
 // CU) for long scans over many tiles (2048^2 x 256 x 1500: 62.9 against 68.0 ms,
 // 1024^2 x 64 x 900: 3.01 against 3.11), else 16 x 16 (four blocks per CU overlap
@@ -603,7 +613,10 @@ bool bpm_shape(int nu, int nv, int nk, int &tile)
     const size_t proj_bytes = 8 * (size_t)bpm_npair(nu) * (size_t)bpm_vp(nv);
     if (nv <= 16 || nk < 32 || 4 * proj_bytes > ((size_t)60 << 20)) return false;
     if ((double)nu * nu * nv * nk < 1.5e9) return false;
-    const long n32 = (long)((nu + 31) / 32) * ((nu + 31) / 32) * ((bpm_vp(nv) / 16 + 3) / 4);
+    const int nzt = bpm_vp(nv) / 16;
+    const long n16 = (long)((nu + 15) / 16) * ((nu + 15) / 16), chunks = nzt % 4 ? 1 : nzt / 4;   // of the smaller launch
+    if (nzt <= 2 ? n16 * nv < 12000 : n16 * chunks < 480) return false;
+    const long n32 = (long)((nu + 31) / 32) * ((nu + 31) / 32) * ((nzt + 3) / 4);
     tile = nk >= 800 && n32 >= 512 ? 32 : 16;
     return true;
 }
@@ -611,7 +624,7 @@ bool bpm_shape(int nu, int nv, int nk, int &tile)
 int run_bpm(const BpmArgs &a, int tile, hipStream_t s)
 {
     // slices in chunks of four tiles of 16, what is left in one chunk of its own
-    const int nzt = (a.nv + 15) / 16, full = nzt / 4, rest = nzt % 4;
+    const int nzt = a.vp / 16, full = nzt / 4, rest = nzt % 4;
     int rc = MR_OK;
     if (full > 0) rc = launch_bpm_tile<4>(a, tile, 0, full, s);
     if (rc == MR_OK && rest == 1) rc = launch_bpm_tile<1>(a, tile, 4 * full, 1, s);
