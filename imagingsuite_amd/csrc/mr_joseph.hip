@@ -721,6 +721,28 @@ int joseph_check(const mr_joseph_geom *g, size_t n_ang)
     return MR_OK;
 }
 
+// Whether a slice count that is no multiple of 16 takes the staged forward (total
+// blocks of slice tiles zt) or joseph_forward_kernel (one wave per 64 rays and 4
+// slices), from what one line of the volume takes with either, in microseconds.
+// A staged block serves 16 bins of the angles of its chunk - 16 where they lie
+// close, one where a wide volume and few angles let no two share a chunk - in
+// the same time, so the number of blocks counts.  The direct kernel's waves all
+// run at once up to one per SIMD (1024), then one after the other, each with the
+// cache misses of its slices.  Fitted to 500 sizes (64^2 to 2048^2, 4 to 60 slices, 8
+// to 360 angles); whole calls, staged / direct, the faster one is taken: 2048^2 x 4 x
+// 60 3.86 / 1.18 ms, 1024^2 x 12 x 20 0.72 / 0.34, 128^2 x 20 x 60 0.082 / 0.061; 300^2 x
+// 20 x 200 0.14 / 0.46, 1024^2 x 12 x 90 1.18 / 1.85, 400^2 x 4 x 180 0.14 / 0.22.
+static bool forward_staged(const mr_joseph_geom &g, size_t n_ang, int zt, long total)
+{
+    if (total < 128) return false;
+    const double blocks = (double)total / 1024.0;
+    const double waves = (double)g.n_det * (double)n_ang * (double)g.nz / (64.0 * 4.0 * 1024.0);
+    const double staged = zt == 8 ? std::max(0.22, 0.32 * blocks) : std::max(0.42, 0.40 * blocks);
+    const double direct =
+        waves <= 1.0 ? 0.28 : std::max(0.45, (0.08 + 0.03 * (double)std::min<size_t>(g.nz, 24)) * waves);
+    return 1.08 * staged < direct;
+}
+
 // Enqueues A (forward) or A^T on s with a resident angle table; no host sync.
 int joseph_launch(const mr_joseph_geom *g, const float *src, float *dst, const JosephDevTables &dt, size_t n_ang,
                   bool forward, hipStream_t s)
@@ -740,11 +762,8 @@ int joseph_launch(const mr_joseph_geom *g, const float *src, float *dst, const J
         const size_t dyn = sizeof(int2) * (g->nx + 3 * R);
         const size_t fixed = sizeof(float) * 2 * R * kFwdW * (zt + 4) + sizeof(float4) * 2 * kFwdKA;
         const int direct = g->nz % 16 == 0 ? 0 : 1;
-        // (Slice counts that are not a multiple of 16 from 128 blocks: with fewer,
-        // joseph_forward_kernel's larger grid wins - 100^2 x 28 x 50, 56 blocks:
-        // 20 against 42 us, 200^2 x 4 x 90, 78: 48 against 46.)
         if (dt.n_chunks > 0 && total < (1L << 31) - 8 && dyn + fixed <= 65536 && g->nx * g->nz < 6500000 &&
-            (!direct || total >= 128)) {
+            (!direct || forward_staged(*g, n_ang, zt, total))) {
             if (zt == 32)
                 hipLaunchKernelGGL((mr::joseph_forward_dma_kernel<32, 1>), grid, dim3(256), dyn, s, a, dt.chunks,
                                    dt.order, dt.n_chunks, nbt, nzs, direct);
@@ -765,6 +784,7 @@ int joseph_launch(const mr_joseph_geom *g, const float *src, float *dst, const J
                                    dt.order, dt.n_chunks, nbt, nzs);
         } else {
             // other slice counts, few blocks or a large volume: direct ray-driven gathers
+            mr::ProfScope gathers("joseph_forward_direct", s);
             dim3 grid((unsigned)((g->n_det + 63) / 64), (unsigned)((n_ang + 3) / 4), (unsigned)(g->nz / ZT));
             hipLaunchKernelGGL(mr::joseph_forward_kernel<ZT>, grid, dim3(256), 0, s, a);
         }
