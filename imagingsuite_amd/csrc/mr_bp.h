@@ -66,7 +66,7 @@ struct BpmArgs {
 bool bpm_shape(int nu, int nv, int nk, int &tile);
 inline int bpm_vp(int nv) { return ((nv & ~3) + 15) & ~15; }
 inline int bpm_npair(int nu) { return (nu + 1) / 2; }
-size_t bpm_part_words(size_t nv, size_t nk);   // words of launch_bp_scale's partial maxima
+size_t bpm_part_words(size_t nv, size_t nk);   // words of launch_bp_scale's maxima and counts
 int launch_bp_scale(const float *proj, const int *idx, const float *wts, int nu, int nv, int nk, unsigned *part,
                     float2 *scale, int *flag, hipStream_t s);
 int launch_bp_split_prep(const BpmArgs &a, const float *proj, const int *idx, const float *wts, int vpad,

@@ -22,10 +22,22 @@
 // reference's float operations, as everywhere.  A group of 4 projections is
 // summed from zero in the matrix unit and added to the voxel's running sum
 // once, against eight fused multiply-adds, so the sum's rounding is smaller
-// than the float kernel's by more than the split adds: error against 64-bit
-// sums of the same samples (relative rms, MFMA / FMA kernel) 1.55e-6 / 1.62e-6
-// at 512^2 x 400 projections, 4.90e-6 / 5.00e-6 at 1024^2 x 1800, equal to
-// three digits where the float positions dominate.
+// than the float kernel's by more than the split adds, as long as the samples
+// of a slice are of similar size: error against 64-bit sums of the same samples
+// (relative rms, MFMA / FMA kernel) 1.55e-6 / 1.62e-6 at 512^2 x 400 projections,
+// 4.90e-6 / 5.00e-6 at 1024^2 x 1800, equal to three digits where the float
+// positions dominate.
+//
+// One sample far above the others (a sentinel for a dead pixel, one projection's
+// weight) takes bits from the rest of its slice: at 1e7 times them the sums' error
+// would be 9 times the float kernel's, at 1e9 600 times.  So a slice of which more
+// than a sixteenth of the samples (those that are not zero; counted on an eighth of
+// them) lie below 2^-17 of the largest does not fit, nor do samples that are not
+// finite or slices whose largest magnitude is outside [2^-63, 2^74):
+// bp_scale_kernel raises a flag on the device, the kernel here leaves without
+// writing and the VALU kernel (gated by the same flag) does the work.  A voxel that
+// only meets such small samples, in a slice that holds few enough of them to
+// fit, has an error of about 2^-40 of the slice's largest per projection.
 //
 // What bounds it: the LDS reads of the windows (2 KB per patch, 16 slices and
 // group: 64 of about 100 cycles per CU), the matrix unit (3 products of 16
@@ -35,11 +47,6 @@
 // bound by that: 2048^2 x 256 x 1500 107 ms, here 55-61 (the clock falls
 // with the samples' toggling); whole FBP of that stack 115 against 69 ms,
 // 701^2 x 37 x 603 1.55 against 0.88.
-//
-// Samples that are not finite, or slices whose largest magnitude is outside
-// [2^-63, 2^74), do not fit that scheme: bp_scale_kernel raises a flag on the
-// device, the kernel here leaves without writing and the VALU kernel (gated
-// by the same flag) does the work.
 #include "mr_bp.h"
 #include "mr_common.h"
 
@@ -58,6 +65,18 @@ typedef unsigned uint4v __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------------------
 // scales and split samples
 // ---------------------------------------------------------------------------
+
+// Largest value and sums over a wave.
+__device__ __forceinline__ unsigned wave_max(unsigned m)
+{
+    for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
+    return m;
+}
+__device__ __forceinline__ unsigned wave_sum(unsigned n)
+{
+    for (int o = 32; o > 0; o >>= 1) n += (unsigned)__shfl_xor((int)n, o);
+    return n;
+}
 
 // part[v][chunk] = largest |proj[idx[k]][v][u] * w[idx[k]]| (its float bits;
 // infinities and NaN compare above every finite value) over one of at most
@@ -85,29 +104,85 @@ __global__ __launch_bounds__(256) void bp_absmax_kernel(const float *__restrict_
             for (int u = lane; u < nu; u += 64) m = max(m, __float_as_uint(row[u] * w) & 0x7fffffffu);
         }
     }
-    for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
+    m = wave_max(m);
     if (lane == 0) red[wv] = m;
     __syncthreads();
     if (threadIdx.x == 0) part[(size_t)v * gridDim.y + blockIdx.y] = max(max(red[0], red[1]), max(red[2], red[3]));
 }
 
+// How wide a slice's range is: behind the maxima of bp_absmax_kernel, part holds
+// per [v][four chunks] how many samples are below 2^-17 of the slice's largest, and
+// how many are not zero, among every eighth run of 64 columns (shifted by a run
+// from one projection to the next, so that all columns take part).
+constexpr unsigned kSmall = 17u << 23;   // 2^-17 in the bits of a float
+__global__ __launch_bounds__(256) void bp_range_kernel(const float *__restrict__ proj, const int *__restrict__ idx,
+                                                       const float *__restrict__ wts, int nu, int nv, int nk, int kc,
+                                                       int nchunk, unsigned *__restrict__ part)
+{
+    __shared__ unsigned red[4][2];
+    const int v = blockIdx.x, k0 = blockIdx.y * 4 * kc, k1 = min(nk, k0 + 4 * kc);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const unsigned m = wave_max(lane < nchunk ? part[(size_t)v * nchunk + lane] : 0u);
+    const unsigned least = m > kSmall ? m - kSmall : 0u;
+    unsigned small = 0, nonzero = 0;
+    for (int k = k0 + wv; k < k1; k += 4) {
+        const int p = idx[k];
+        const float w = wts[p];
+        const float *row = proj + ((size_t)p * nv + v) * nu;
+        for (int u = 64 * (k & 7) + lane; u < nu; u += 512) {
+            const unsigned x = __float_as_uint(row[u] * w) & 0x7fffffffu;
+            small += x != 0 && x < least ? 1u : 0u;
+            nonzero += x != 0 ? 1u : 0u;
+        }
+    }
+    small = wave_sum(small);
+    nonzero = wave_sum(nonzero);
+    if (lane == 0) {
+        red[wv][0] = small;
+        red[wv][1] = nonzero;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+        part[(size_t)nv * nchunk + ((size_t)threadIdx.x * nv + v) * gridDim.y + blockIdx.y] =
+            red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
+}
+
 // scale[v] = (factor on the samples of slice v, its inverse); *flag = 1 when
-// some slice does not fit the split (not finite, or outside the exponent
-// range).  One block.
+// some slice does not fit the split: not finite, outside the exponent range, or
+// more than a sixteenth of its samples below 2^-17 of its largest.  One block, 16
+// lanes per slice (one lane: 22 us at 256 slices, against 6).
 __global__ __launch_bounds__(1024) void bp_scale_kernel(const unsigned *__restrict__ part, int nv, int nchunk,
                                                         float2 *__restrict__ scale, int *__restrict__ flag)
 {
+    const int lane = threadIdx.x & 15;
+    const int nrange = (nchunk + 3) / 4;   // at most 16
     int bad = 0;
-    for (int v = threadIdx.x; v < nv; v += 1024) {
-        unsigned m = 0;
-        for (int c = 0; c < nchunk; ++c) m = max(m, part[(size_t)v * nchunk + c]);
+    for (int v0 = 0; v0 < nv; v0 += 64) {
+        const int v = v0 + (threadIdx.x >> 4);
+        unsigned m = 0, small = 0, nonzero = 0;
+#pragma unroll
+        for (int i = 0; i < kScaleChunks / 16; ++i) {
+            const int c = lane + 16 * i;
+            if (v >= nv || c >= nchunk) continue;
+            m = max(m, part[(size_t)v * nchunk + c]);
+        }
+        if (v < nv && lane < nrange) {
+            const unsigned *counts = part + (size_t)nv * nchunk + (size_t)v * nrange + lane;
+            small = counts[0];
+            nonzero = counts[(size_t)nv * nrange];
+        }
+        for (int o = 8; o > 0; o >>= 1) {
+            m = max(m, (unsigned)__shfl_xor((int)m, o));
+            small += (unsigned)__shfl_xor((int)small, o);
+            nonzero += (unsigned)__shfl_xor((int)nonzero, o);
+        }
         const int e = (int)(m >> 23);   // biased exponent of the largest magnitude
         float2 s = make_float2(1.0f, 1.0f);
         if (m != 0) {
-            if (e < 64 || e > 200) bad = 1;
+            if (e < 64 || e > 200 || small > nonzero / 16) bad = 1;
             else s = make_float2(__uint_as_float((unsigned)(268 - e) << 23), __uint_as_float((unsigned)(e - 14) << 23));
         }
-        scale[v] = s;
+        if (lane == 0 && v < nv) scale[v] = s;
     }
     bad = __syncthreads_or(bad);
     if (threadIdx.x == 0) *flag = bad;
@@ -559,7 +634,7 @@ static int scale_chunks(size_t nk, int &kc)
 size_t bpm_part_words(size_t nv, size_t nk)
 {
     int kc;
-    return nv * (size_t)scale_chunks(nk, kc);
+    return 3 * nv * (size_t)scale_chunks(nk, kc);
 }
 
 int launch_bp_scale(const float *proj, const int *idx, const float *wts, int nu, int nv, int nk, unsigned *part,
@@ -570,6 +645,8 @@ int launch_bp_scale(const float *proj, const int *idx, const float *wts, int nu,
     const int nchunk = scale_chunks((size_t)nk, kc);
     hipLaunchKernelGGL(bp_absmax_kernel, dim3((unsigned)nv, (unsigned)nchunk), dim3(256), 0, s, proj, idx, wts, nu, nv,
                        nk, kc, part);
+    hipLaunchKernelGGL(bp_range_kernel, dim3((unsigned)nv, (unsigned)((nchunk + 3) / 4)), dim3(256), 0, s, proj, idx,
+                       wts, nu, nv, nk, kc, nchunk, part);
     hipLaunchKernelGGL(bp_scale_kernel, dim3(1), dim3(1024), 0, s, part, nv, nchunk, scale, flag);
     MR_HIP(hipGetLastError());
     return MR_OK;

@@ -155,9 +155,10 @@ class BackProjector:
     (ROI-relative), ``direction`` 0 = CW, 1 = CCW, ``buffer_size`` is
     ProjectionBufferSize (16 reproduces the reference exactly, including its
     dropped projections; 0 back-projects every projection).  ``fused`` folds
-    the interpolation into fused multiply-adds or, for large stacks, runs it on
-    the matrix cores in split halves (float rounding differs from the
-    reference; otherwise results are bit-identical).
+    the interpolation into fused multiply-adds or, for large stacks whose
+    samples are of similar size, runs it on the matrix cores in split halves
+    (float rounding differs from the reference, and between a stack and its
+    slabs; otherwise results are bit-identical).
 
     ``correct_tilt`` runs the module's bCorrectTilt branch with
     ``tilt_angle`` (degrees) and ``tilt_pivot`` (detector row); ``row0`` is

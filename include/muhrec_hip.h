@@ -117,7 +117,16 @@ typedef struct {
                             results); 1: float rounding only: interpolation folded into
                             fused multiply-adds, or for large stacks (17 slices or more,
                             see mr_bp_plan_kernel) on the matrix cores with every factor
-                            split into two halves, at least as near to double */
+                            split into two halves: measured as near to double as the
+                            former for samples of similar size.  Stacks with samples that
+                            are not finite, or with a slice of which more than a sixteenth
+                            of the samples lie below 2^-17 of its largest, take the fused
+                            multiply-adds; in the other slices a sample holds 22 bits, or an
+                            absolute 2^-40 of the slice's largest where that is more.
+                            Which of the two runs depends on the whole call: its size, all
+                            its samples, and accumulation (always multiply-adds), so a
+                            stack cut into slabs or into accumulating calls agrees with
+                            one call to rounding, not in every bit */
     /* Axis-tilt correction, the bCorrectTilt branches of the three back-projectors
      * (MultiProjBPparallel.cpp:49-114, MultiProjBP.cpp:50-96, NNMultiProjBP.cpp:48-81)
      * and the mask shrink of BuildCircleMask (BackProjectorModuleBase.cpp:171-180).
