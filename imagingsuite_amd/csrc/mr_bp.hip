@@ -1321,6 +1321,7 @@ struct mr_bp_plan {
     void *d_split = nullptr;
     size_t split_cap = 0;                 // bytes
     bool no_split = false;                // the split samples did not fit the memory: VALU kernel
+    bool accumulated = false;             // the last call accumulated: VALU kernel
 };
 
 namespace mr {
@@ -1483,8 +1484,8 @@ extern "C" int mr_bp_plan_kernel(const mr_bp_plan *plan, char *name, size_t len)
     mr::clear_error();
     MR_REQUIRE(plan != nullptr && name != nullptr && len > 0, "NULL argument");
     int tile = 0;
-    // with tables loaded, the form their projection count selects
-    const std::string d = plan->loaded && mr::plan_bpm(plan, plan->loaded_nk, tile)
+    // with tables loaded, the form that their projection count and the last call select
+    const std::string d = plan->loaded && !plan->accumulated && mr::plan_bpm(plan, plan->loaded_nk, tile)
                               ? "bp_mfma_kernel tile=" + std::to_string(tile)
                               : mr::describe_bp((int)plan->p.width, (int)plan->p.slices,
                                                 plan->loaded ? (int)plan->loaded_nk : 0, plan->p.interp, plan->impl,
@@ -1563,6 +1564,7 @@ int bp_enqueue(mr_bp_plan *plan, const float *d_proj, float *d_volume, int accum
     int tile = 0;
     // accumulation onto a volume keeps the VALU kernel, whose running sum
     // starts from the volume
+    plan->accumulated = accumulate != 0;
     const bool bpm = !accumulate && plan_bpm(plan, nk, tile);
     int *flag = nullptr;
     if (bpm) {

@@ -149,8 +149,9 @@ int mr_bp_plan_destroy(mr_bp_plan *plan);
 /* Name of the kernel variant mr_bp_parallel launches for this plan (slice
  * tile, projection chunk, block order), e.g.
  * "bp_lds_kernel<32,0,false,4,1> order=1 sw=4".  Once the plan has projected,
- * the variant that its number of projections selects: also
- * "bp_mfma_kernel tile=32" (fused plans) and the thin tiles of small grids.
+ * the variant of the last call: also "bp_mfma_kernel tile=32" (fused plans, calls
+ * that do not accumulate; whether the samples then fit is known on the device
+ * only) and the thin tiles of small grids.
  * Diagnostics only; no counterpart in the reference. */
 int mr_bp_plan_kernel(const mr_bp_plan *plan, char *name, size_t len);
 /* Host copy of the circle mask: for row y the voxels first[y] <= x < second[y]

@@ -59,3 +59,18 @@ def test_ragged_ends(dev, monkeypatch, nu, nv, n_p):
     monkeypatch.setenv("MR_BP_STAGE64", "1")
     b = BackProjector("MultiProjBPparallel", nu, nv, nu / 2 + 1.25, buffer_size=0, fused=True).process(t, ang, w)
     assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+def test_plan_reports_the_last_call(dev):
+    """Accumulating calls run on the vector kernel, and the plan says so."""
+    from imagingsuite_amd.recon import BackProjector
+    nu, nv, n_p = 512, 32, 200
+    bp = BackProjector("MultiProjBPparallel", nu, nv, nu / 2, buffer_size=0, fused=True)
+    t = torch.ones((n_p, nv, nu), dtype=torch.float32, device=dev)
+    ang, w = np.arange(n_p, dtype=np.float32), np.ones(n_p, np.float32)
+    vol = bp.process(t, ang, w)
+    assert bp.kernel.startswith("bp_mfma_kernel")
+    bp.process(t, ang, w, volume=vol, accumulate=True)
+    assert bp.kernel.startswith("bp_lds_kernel")
+    bp.process(t, ang, w, volume=vol)
+    assert bp.kernel.startswith("bp_mfma_kernel")
