@@ -41,9 +41,9 @@ void bp_set_tilt_row0(mr_bp_plan *plan, size_t row0);
 size_t bp_plan_width(const mr_bp_plan *plan);
 
 // sino[k][u][v] = proj[idx[k]][v][u] * wts[idx[k]] for the nk used
-// projections (v < nv; zero for nv <= v < vpad).
+// projections (v < nv; zero for nv <= v < vpad).  gate: only if *gate != 0.
 int launch_bp_prep(const float *proj, float *sino, const int *idx, const float *wts, int nu, int nv,
-                   int vpad, int nk, hipStream_t s);
+                   int vpad, int nk, hipStream_t s, const int *gate = nullptr);
 // Back-projection kernel for one stack.  impl 0: direct gathers (MultiProjBP
 // with slices % 4 != 0, whose second column is read at a different offset);
 // 1: LDS-staged tiles.  exact: the reference's float operation order.
@@ -58,6 +58,7 @@ struct BpmArgs {
     const float2 *scale;     // per slice: factor on the samples, its inverse
     const int *flag;         // set: the samples do not fit the split, the kernel leaves at once
     int nu, nv, vp, npair, nk, nz4;   // vp: slices of whole groups of four, rounded up to 16; npair: column pairs
+    int nvs;                 // slices of the projections and of the volume in memory (nv, or more for a slab of them)
     int chain;               // 1: the volume holds the sums of earlier projections, continue them
     int ntx, nty, ntz, zt0, sw;
 };

@@ -35,8 +35,9 @@ __global__ __launch_bounds__(256) void bp_prep_kernel(const float *__restrict__ 
                                                       float *__restrict__ sino,
                                                       const int *__restrict__ idx,
                                                       const float *__restrict__ wts, int nu, int nv,
-                                                      int vpad)
+                                                      int vpad, const int *__restrict__ gate)
 {
+    if (gate && *gate == 0) return;
     __shared__ float tile[32][33];
     const int k = blockIdx.z;
     const int p = idx[k];
@@ -63,8 +64,9 @@ __global__ __launch_bounds__(256) void bp_prep4_kernel(const float *__restrict__
                                                        float *__restrict__ sino,
                                                        const int *__restrict__ idx,
                                                        const float *__restrict__ wts, int nu, int nv,
-                                                       int vpad)
+                                                       int vpad, const int *__restrict__ gate)
 {
+    if (gate && *gate == 0) return;
     __shared__ float tile[64][65];
     const int k = blockIdx.z;
     const int p = idx[k];
@@ -95,15 +97,15 @@ __global__ __launch_bounds__(256) void bp_prep4_kernel(const float *__restrict__
 
 // Weighting and transposition of the used projections into the sinogram.
 int launch_bp_prep(const float *proj, float *sino, const int *idx, const float *wts, int nu, int nv,
-                          int vpad, int nk, hipStream_t s)
+                          int vpad, int nk, hipStream_t s, const int *gate)
 {
     ProfScope prof("bp_prep", s);
     if (nu % 4 == 0) {
         dim3 g((unsigned)((nu + 63) / 64), (unsigned)((vpad + 63) / 64), (unsigned)nk);
-        hipLaunchKernelGGL(bp_prep4_kernel, g, dim3(256), 0, s, proj, sino, idx, wts, nu, nv, vpad);
+        hipLaunchKernelGGL(bp_prep4_kernel, g, dim3(256), 0, s, proj, sino, idx, wts, nu, nv, vpad, gate);
     } else {
         dim3 g((unsigned)((nu + 31) / 32), (unsigned)((vpad + 31) / 32), (unsigned)nk);
-        hipLaunchKernelGGL(bp_prep_kernel, g, dim3(256), 0, s, proj, sino, idx, wts, nu, nv, vpad);
+        hipLaunchKernelGGL(bp_prep_kernel, g, dim3(256), 0, s, proj, sino, idx, wts, nu, nv, vpad, gate);
     }
     MR_HIP(hipGetLastError());
     return MR_OK;
@@ -1574,7 +1576,7 @@ int bp_enqueue(mr_bp_plan *plan, const float *d_proj, float *d_volume, int accum
         flag = reinterpret_cast<int *>(part + mr::bpm_part_words(q.slices, nk));
         m.split = reinterpret_cast<const unsigned *>(plan->d_sino);
         m.vol = d_volume; m.tab = plan->d_tab; m.mask = plan->d_mask; m.scale = scale; m.flag = flag;
-        m.nu = (int)q.width; m.nv = (int)q.slices; m.vp = mr::bpm_vp(m.nv); m.npair = mr::bpm_npair(m.nu);
+        m.nu = (int)q.width; m.nv = m.nvs = (int)q.slices; m.vp = mr::bpm_vp(m.nv); m.npair = mr::bpm_npair(m.nu);
         m.nk = (int)nk; m.nz4 = (int)((q.slices / 4) * 4);
         int rc = mr::launch_bp_scale(d_proj, plan->d_idx, plan->d_w, m.nu, m.nv, m.nk, part, scale, flag, s);
         if (rc == MR_OK) rc = mr::launch_bp_split_prep(m, d_proj, plan->d_idx, plan->d_w, (int)plan->vpad, s);
@@ -2095,7 +2097,7 @@ extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *
             mr::BpmArgs &q = b.margs;
             q.split = reinterpret_cast<const unsigned *>(b.d_sino);
             q.vol = d.d_volume; q.tab = b.d_tab; q.mask = b.d_mask; q.scale = b.d_scale; q.flag = p->d_flags + i;
-            q.nu = a.nu; q.nv = a.nv; q.vp = mr::bpm_vp(a.nv); q.npair = mr::bpm_npair(a.nu);
+            q.nu = a.nu; q.nv = q.nvs = a.nv; q.vp = mr::bpm_vp(a.nv); q.npair = mr::bpm_npair(a.nu);
             q.nk = a.nk; q.nz4 = a.nz4;
             a.gate = q.flag;   // the single-stack launch behind the matrix-core one
         }

@@ -223,14 +223,14 @@ __global__ __launch_bounds__(256) void bp_split_prep_kernel(const float *__restr
                                                             const int *__restrict__ idx,
                                                             const float *__restrict__ wts,
                                                             const float2 *__restrict__ scale,
-                                                            const int *__restrict__ flag, int nu, int nv, int nz4,
-                                                            int vpad, int vp, int npair)
+                                                            const int *__restrict__ flag, int nu, int nv, int nvs,
+                                                            int nz4, int vpad, int vp, int npair)
 {
     __shared__ float tile[64][65];
     const int k = blockIdx.z, p = idx[k];
     const float w = wts[p];
     const int u0 = blockIdx.x * 64, v0 = blockIdx.y * 64;
-    const float *src = proj + (size_t)p * nu * nv;
+    const float *src = proj + (size_t)p * nu * nvs;
     if ((nu & 3) == 0) {
         const int c4 = threadIdx.x & 15, rr = threadIdx.x >> 4;
 #pragma unroll
@@ -376,7 +376,7 @@ __device__ __forceinline__ void bpm_tile(const BpmArgs &a, int bx, int by, int b
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     if (y < a.nu && x + i < a.nu && z < a.nv)
-                        acc[q][zt][i] = a.vol[((size_t)y * a.nu + x + i) * a.nv + z] * a.scale[z].x;
+                        acc[q][zt][i] = a.vol[((size_t)y * a.nu + x + i) * a.nvs + z] * a.scale[z].x;
             }
     }
 
@@ -578,7 +578,7 @@ __device__ __forceinline__ void bpm_tile(const BpmArgs &a, int bx, int by, int b
         for (int i = 0; i < 4; ++i) {
             if (x + i >= a.nu) continue;
             const bool in = x + i >= mk.x && x + i < mk.y;
-            float *out = a.vol + ((size_t)y * a.nu + x + i) * a.nv + z0 + m;
+            float *out = a.vol + ((size_t)y * a.nu + x + i) * a.nvs + z0 + m;
 #pragma unroll
             for (int zt = 0; zt < NT; ++zt)
                 if (z0 + 16 * zt + m < a.nv) out[16 * zt] = in ? acc[q][zt][i] * inv[zt] : 0.0f;
@@ -659,7 +659,7 @@ int launch_bp_split_prep(const BpmArgs &a, const float *proj, const int *idx, co
     // (vpad, the float sinogram's slices, exceeds vp where nv % 16 is 1, 2 or 3)
     dim3 g((unsigned)((2 * a.npair + 63) / 64), (unsigned)((std::max(a.vp, vpad) + 63) / 64), (unsigned)a.nk);
     hipLaunchKernelGGL(bp_split_prep_kernel, g, dim3(256), 0, s, proj, const_cast<unsigned *>(a.split), idx, wts,
-                       a.scale, a.flag, a.nu, a.nv, a.nz4, vpad, a.vp, a.npair);
+                       a.scale, a.flag, a.nu, a.nv, a.nvs, a.nz4, vpad, a.vp, a.npair);
     MR_HIP(hipGetLastError());
     return MR_OK;
 }

@@ -21,8 +21,8 @@
 // order (the kernels load the voxel, add the chunk's projections in order
 // and store it), so the result equals mr_bp_parallel's bit for bit.  In the
 // matrix-core form the samples' scale comes from all projections before the
-// first chunk, chunks are whole groups of four projections and a chunk
-// continues the sums of the ones before it: the same bits again.
+// first chunk, chunks are whole groups of four projections of a slab of slices
+// and a chunk continues the sums of the ones before it: the same bits again.
 //
 // The host tables reach the scratch through kernel arguments (scratch_put_kernel),
 // so no host buffer has to outlive the call and nothing is allocated.
@@ -177,20 +177,44 @@ extern "C" int mr_bp_parallel_noalloc(const mr_bp_params *params, const float *d
     const bool bpm = q.fused && !accumulate && q.interp == MR_INTERP_LINEAR && impl == 1 &&
                      mr::bpm_shape((int)q.width, (int)q.slices, (int)nk, tile);
     mr::BpmArgs m{};
-    size_t kc_max = sino_bytes / proj_bytes;
+    const size_t kc_max = sino_bytes / proj_bytes;
     if (bpm) {
         float2 *scale = reinterpret_cast<float2 *>(base + off_scale);
         int *flag = reinterpret_cast<int *>(base + off_flag);
         m.split = reinterpret_cast<const unsigned *>(d_sino);
-        m.vol = d_volume; m.mask = d_mask; m.scale = scale; m.flag = flag;
-        m.nu = (int)q.width; m.nv = (int)q.slices; m.vp = mr::bpm_vp(m.nv); m.npair = mr::bpm_npair(m.nu);
-        m.nz4 = (int)((q.slices / 4) * 4);
-        // groups of four that fit as split or as float samples (at least one: bpm_shape)
-        kc_max = std::min(kc_max, sino_bytes / (8 * (size_t)m.npair * (size_t)m.vp)) / 4 * 4;
+        m.mask = d_mask; m.flag = flag;
+        m.nu = (int)q.width; m.nvs = (int)q.slices; m.npair = mr::bpm_npair(m.nu);
         MR_REQUIRE(mr::bpm_part_words(q.slices, nk) * sizeof(unsigned) <= sino_bytes, "slices exceed the fixed scratch");
-        rc = mr::launch_bp_scale(d_proj, d_idx, d_w, m.nu, m.nv, (int)nk, reinterpret_cast<unsigned *>(d_sino), scale,
+        rc = mr::launch_bp_scale(d_proj, d_idx, d_w, m.nu, m.nvs, (int)nk, reinterpret_cast<unsigned *>(d_sino), scale,
                                  flag, s);
         if (rc != MR_OK) return rc;
+        // Every chunk reads and writes the volume of its slices, so the slices go
+        // in slabs (whole slice chunks of run_bpm: the same bits) of which 32
+        // projections or all fit (2048^2 x 1024 x 40 in one slab, 4 projections a
+        // chunk, 122 ms; in slabs of 192 slices, 40 projections, 11 ms).
+        const size_t want = std::min<size_t>(32, (nk + 3) / 4 * 4);
+        auto fit = [&](size_t slices) {   // whole groups of four, as split or as float samples
+            return std::min(sino_bytes / (8 * (size_t)m.npair * (size_t)mr::bpm_vp((int)slices)),
+                            sino_bytes / (q.width * ((slices + 3) & ~size_t(3)) * sizeof(float))) / 4 * 4;
+        };
+        size_t slab = q.slices;
+        if (fit(slab) < want)
+            for (slab = (q.slices - 1) / 64 * 64; slab > 64 && fit(slab) < want;) slab -= 64;
+        const size_t nz4 = (q.slices / 4) * 4;
+        for (size_t z = 0; z < nz4; z += slab) {
+            const size_t left = q.slices - z, n = left - std::min(left, slab) < 4 ? left : slab;
+            m.vol = d_volume + z; m.scale = scale + z;
+            m.nv = (int)n; m.vp = mr::bpm_vp(m.nv); m.nz4 = m.nv / 4 * 4;
+            for (size_t kb = 0; kb < nk; kb += (size_t)m.nk) {
+                m.tab = d_tab + kb;
+                m.nk = (int)std::min(fit(n), nk - kb);
+                m.chain = kb > 0 ? 1 : 0;
+                rc = mr::launch_bp_split_prep(m, d_proj + z * q.width, d_idx + kb, d_w, (m.nv + 3) & ~3, s);
+                if (rc == MR_OK) rc = mr::run_bpm(m, tile, s);
+                if (rc != MR_OK) return rc;
+            }
+            if (n == left) break;
+        }
     }
 
     mr::BpArgs a{};
@@ -203,20 +227,14 @@ extern "C" int mr_bp_parallel_noalloc(const mr_bp_params *params, const float *d
     a.nz4 = (int)((q.slices / 4) * 4);
     a.bstride = q.multiprojbp ? a.nz4 : (int)vpad;
     a.gate = m.flag;
-    // nk == 0 still runs one launch: it writes the zeroed (or unchanged) volume
+    // With the matrix-core form these run only if it left (its flag).  nk == 0 still
+    // runs one launch: it writes the zeroed (or unchanged) volume
     size_t kb = 0;
     do {
         const size_t kc = std::min(kc_max, nk - kb);
-        if (bpm) {
-            m.tab = d_tab + kb;
-            m.nk = (int)kc;
-            m.chain = kb > 0 ? 1 : 0;
-            rc = mr::launch_bp_split_prep(m, d_proj, d_idx + kb, d_w, (int)vpad, s);
-            if (rc == MR_OK) rc = mr::run_bpm(m, tile, s);
-            if (rc != MR_OK) return rc;
-        } else if (kc > 0) {
+        if (kc > 0) {
             rc = mr::launch_bp_prep(d_proj, d_sino, d_idx + kb, d_w, (int)q.width, (int)q.slices, (int)vpad,
-                                    (int)kc, s);
+                                    (int)kc, s, m.flag);
             if (rc != MR_OK) return rc;
         }
         a.tab = d_tab + kb;
