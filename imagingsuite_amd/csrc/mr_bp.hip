@@ -2019,14 +2019,14 @@ int occupancy_grid(int &grid, int exact)
 
 }  // namespace
 
-extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *stacks, size_t n_stacks,
-                                    int flags)
+namespace {
+
+// mr_batch_plan_create; matrix: larger fused stacks may take the matrix-core form
+// (left true if one did).
+int batch_create(mr_batch_plan **plan, const mr_batch_stack *stacks, size_t n_stacks, int flags, bool &matrix)
 {
-    MR_GUARD_BEGIN
-    mr::clear_error();
-    MR_REQUIRE(plan != nullptr && stacks != nullptr && n_stacks > 0, "NULL argument or empty batch");
-    MR_REQUIRE((flags & ~(MR_BATCH_TUNE | MR_BATCH_FUSED)) == 0, "unknown batch flags");
-    *plan = nullptr;
+    const bool allowed = matrix;
+    matrix = false;
     const bool tune = (flags & MR_BATCH_TUNE) != 0;
     auto *p = new mr_batch_plan();
     p->exact = (flags & MR_BATCH_FUSED) ? 0 : 1;
@@ -2066,7 +2066,8 @@ extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *
             m[y].x = (int)first[y];
             m[y].y = (int)std::max(first[y], second[y]);
         }
-        b.bpm = !p->exact && mr::bpm_shape((int)d.width, (int)d.slices, (int)b.n_used, b.tile);
+        b.bpm = allowed && !p->exact && mr::bpm_shape((int)d.width, (int)d.slices, (int)b.n_used, b.tile);
+        matrix = matrix || b.bpm;
         size_t sino = std::max<size_t>(b.n_used, 1) * d.width * b.vpad;
         if (b.bpm)
             sino = std::max(sino, b.n_used * 2 * (size_t)mr::bpm_npair((int)d.width) * mr::bpm_vp((int)d.slices));
@@ -2202,6 +2203,28 @@ extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *
     }
     *plan = p;
     return MR_OK;
+}
+
+}  // namespace
+
+extern "C" int mr_batch_plan_create(mr_batch_plan **plan, const mr_batch_stack *stacks, size_t n_stacks,
+                                    int flags)
+{
+    MR_GUARD_BEGIN
+    mr::clear_error();
+    MR_REQUIRE(plan != nullptr && stacks != nullptr && n_stacks > 0, "NULL argument or empty batch");
+    MR_REQUIRE((flags & ~(MR_BATCH_TUNE | MR_BATCH_FUSED)) == 0, "unknown batch flags");
+    *plan = nullptr;
+    bool matrix = true;
+    int rc = batch_create(plan, stacks, n_stacks, flags, matrix);
+    if (rc == MR_ERR_HIP && matrix) {
+        // the split samples take more memory than float ones: the latter may fit
+        (void)hipGetLastError();
+        mr::clear_error();
+        matrix = false;
+        rc = batch_create(plan, stacks, n_stacks, flags, matrix);
+    }
+    return rc;
     MR_GUARD_END
 }
 
