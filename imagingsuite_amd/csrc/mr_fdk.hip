@@ -716,7 +716,7 @@ struct mr_fdk_plan {
     double mask_radius = 0.0;   // farthest voxel of the mask from the rotation axis
     float *d_imgt = nullptr;    // transposed projections of the slice-lane kernel
     size_t imgt_cap = 0;        // floats
-    bool no_slice = false;      // column-thread kernel only (MR_FDK_COLUMN, or no memory for the copy)
+    bool no_slice = false;      // column-thread kernel only (MR_FDK_COLUMN)
     size_t cap_np = 0;
 };
 
@@ -1105,8 +1105,7 @@ extern "C" int mr_fdk_bp(mr_fdk_plan *plan, float *d_proj, size_t n_proj, size_t
             if (hipMalloc(&plan->d_imgt, need * sizeof(float)) == hipSuccess) plan->imgt_cap = need;
             else {
                 (void)hipGetLastError();
-                plan->d_imgt = nullptr;
-                plan->no_slice = true;
+                plan->d_imgt = nullptr;   // this call on the column kernel; the next one tries again
             }
         }
         if (plan->d_imgt) {

@@ -352,7 +352,11 @@ int mr_fdk_plan_window(const mr_fdk_plan *plan, size_t *cbct_roi);
 /* d_proj: [n_proj][win_rows][width] raw projections of the window (device,
  * used as scratch: it is weighted and filtered in place).  d_volume:
  * [nz][nx][nx] (MatrixXYZ, x fastest) with nx = roi[2]-roi[0], nz = roi[3]-roi[1];
- * overwritten with the mirrored/flipped result (fdkreconbase.cpp:259-270). */
+ * overwritten with the mirrored/flipped result (fdkreconbase.cpp:259-270).
+ * Volumes from 512 x 512 x 224 may take a kernel that reads a transposed copy
+ * of the projections (n_proj x width x (win_rows + the rows that a block of 256
+ * slices spans) floats).  The plan keeps that copy until it is destroyed; a call
+ * for which it cannot be allocated runs without it, with the same results. */
 int mr_fdk_bp(mr_fdk_plan *plan, float *d_proj, size_t n_proj, size_t win_rows,
               const float *angles, const float *weights, float *d_volume, void *stream);
 

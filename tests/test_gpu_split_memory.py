@@ -1,8 +1,9 @@
-"""GPU: fused stacks whose split samples do not fit the device's free memory.
+"""GPU: calls whose fast form needs a copy that does not fit the device's free memory.
 
 The matrix-core form pads slices to 16 (20 slices: 32, float samples 20).  Where
 only the float samples fit, plans and batches run on the vector kernel, with its
-bits, instead of failing.
+bits, instead of failing.  An FDK plan that had no room for its transposed
+projections makes the copy at the next call that has.
 """
 import numpy as np
 import pytest
@@ -88,3 +89,28 @@ def test_batch_falls_back(dev, monkeypatch):
     br.close()
     # with room the same stacks run on the matrix cores
     assert BatchReconstructor(stacks, tune=False, fused=True).slice_tile == 64
+
+
+def test_fdk_plan_takes_its_copy_later(dev):
+    from imagingsuite_amd import _lib
+    from imagingsuite_amd.recon import FDKbp_single
+    n, rows, n_p = 512, 256, 400
+    copy = 4 * n_p * n * rows          # without the rows behind the window
+    fdk = FDKbp_single(500.0, 1000.0, (0.2, 0.2), (0.1, 0.1, 0.1), (n / 2, rows / 2), n / 2, (0, 0, n, rows), n - 1)
+    proj = torch.randn((n_p, rows, n), device=dev, generator=torch.Generator(device=dev).manual_seed(7))
+    angles = (np.arange(n_p) * (360.0 / n_p)).astype(np.float32)
+    weights = np.full(n_p, 1.0 / n_p, np.float32)
+    vols = [torch.empty((rows, n, n), device=dev) for _ in range(2)]
+    work = [proj.clone(), proj]
+    launches = []
+    rest = _squeeze(dev, SLACK, copy)
+    for w, v in zip(work, vols):
+        _lib.profile(True)
+        _lib.profile_reset()
+        fdk.process(w, angles, weights, volume=v)
+        launches.append(_lib.profile_query("fdk_transpose")[1])
+        _lib.profile(False)
+        rest = None
+        torch.cuda.empty_cache()
+    assert launches == [0, 1]
+    assert torch.equal(vols[0], vols[1])
