@@ -614,17 +614,18 @@ def fdk_leg(steps, full):
             m.process(work, angles, weights, vol)
         step()
         ms, k = profiled(lambda: timed_staged(staged, lambda w: m.process(w, angles, weights, vol), step, nsteps,
-                                              name), [kname, "row_filter"])
+                                              name), [kname, "row_filter", "fdk_transpose"])
         return ms, k
 
     ms, k = run_module(fdk, "fdk", "fdk_bp", steps)
     kms = k["fdk_bp"][0]
-    kname = "fdk_kernel<16,false>"
+    kname = "fdk_slice_kernel<false>" if k["fdk_transpose"][1] else "fdk_kernel<16,false>"
     traffic, l2 = profile_counters("fdk_traffic_c3.json", kname)
     out = {"workload": "FDK 1024^3 from 720 projections, 1024^2 detector at 0.2 mm, SOD 500, SDD 1000",
            "filter": "Shepp-Logan + cosine pre-weighting", "precision": "exact positions",
            "ms_per_step": round(ms, 3), "GUPS": round(updates / (ms / 1e3) / 1e9, 2),
-           "kernels_ms": {"row_filter_fdk": round(k["row_filter"][0], 3), "fdk_bp": round(kms, 3)},
+           "kernels_ms": {"row_filter_fdk": round(k["row_filter"][0], 3),
+                          "fdk_transpose": round(k["fdk_transpose"][0], 3), "fdk_bp": round(kms, 3)},
            "input": staged.note()}
     out["roofline"] = roofline(kname, kms, updates, FDK_FLOP_PER_UPDATE,
                                alg_bytes=4.0 * (n * (cb[3] - cb[1]) * n_p + n ** 3), traffic=traffic, l2_bytes=l2)
