@@ -311,13 +311,20 @@ __global__ __launch_bounds__(256) void bp_tilt_kernel(BpArgs a)
 // every thread gathers its two columns from LDS with 16-byte reads.  Rows of
 // the staged tile are ZT+4 floats apart, which spreads 16 distinct columns over
 // distinct LDS banks.  Two buffers of C projections (KC of them where two fit
-// beside enough blocks, else KC / 2): direct loads fill one while the other is
-// summed, one barrier per chunk; the lowest columns of 64 projections are
-// computed at once, one per lane.  (Staged through registers between two
-// barriers, lowest columns in LDS: exact 1024^2 x 32 x 625 2.06 against 1.89 ms,
-// nearest neighbour 512^2 x 64 x 200 0.224 against 0.171, tilted 1024^2 x 64 x 300
-// 2.27 against 2.11.)  Bound by the LDS reads, 8 bytes per voxel, slice and
-// projection: 1.8 of the 1.89 ms at 128 bytes per cycle and CU.
+// beside enough blocks, else KC / 2): the direct loads of the next chunk are
+// issued ahead of a chunk's sums, one barrier per chunk; the lowest columns of 64
+// projections are computed at once, one per lane.  (Staged through registers
+// between two barriers, lowest columns in LDS: exact 1024^2 x 32 x 625 2.06 against
+// 1.89 ms, nearest neighbour 512^2 x 64 x 200 0.224 against 0.171, tilted 1024^2 x 64
+// x 300 2.27 against 2.11.)  The compiler, which cannot tell the buffers apart,
+// waits for those loads ahead of the chunk's first LDS read, so it is the CU's
+// other blocks that they overlap with; reads that do not wait took 13 registers
+// more and the same time (306 sizes, 0.92 to 1.12, mean 1.00).
+// No unit bounds it alone.  Reference order, 1024^2 x 32 x 625, 1.85 ms: the LDS
+// reads (two of 16 bytes per four updates, no bank conflicts) keep the LDS busy
+// for 51 % of the cycles, a SIMD issues 0.29 vector instructions per cycle (at
+// 2.35 cycles each two thirds of the time), and 31 % of the wave cycles wait.
+// Tilted, 1024^2 x 64 x 900, 6.4 ms, one projection at a time: 43 %, 0.29, 38 %.
 // EXACT = true keeps the reference's float operation order per voxel
 // (bit-identical); EXACT = false folds the interpolation into two FMAs.
 constexpr int kBpSpan = 26;

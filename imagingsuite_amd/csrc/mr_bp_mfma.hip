@@ -39,14 +39,15 @@
 // only meets such small samples, in a slice that holds few enough of them to
 // fit, has an error of about 2^-40 of the slice's largest per projection.
 //
-// What bounds it: the LDS reads of the windows (2 KB per patch, 16 slices and
-// group: 64 of about 100 cycles per CU), the matrix unit (3 products of 16
-// cycles per wave) and the VALU (weights: about 40 instructions per patch,
-// which the matrix unit overlaps only in part) are all above half busy.
-// bp_lds_kernel reads two 16-byte vectors from LDS for four updates and is
-// bound by that: 2048^2 x 256 x 1500 107 ms, here 55-61 (the clock falls
-// with the samples' toggling); whole FBP of that stack 115 against 69 ms,
-// 701^2 x 37 x 603 1.55 against 0.88.
+// What bounds it (2048^2 x 256 x 1500): the LDS reads of the windows (2 KB per
+// patch, 16 slices and group) keep the LDS busy for 67 % of the cycles, the matrix
+// unit (3 products of 16 cycles per wave) is busy for 45 %, the VALU (weights:
+// about 40 instructions per patch) issues 0.16 instructions per cycle and SIMD,
+// and 40 % of the wave cycles wait for one of them.  bp_lds_kernel takes 107 ms
+// for it, this one 60-64 (the clock falls with the samples' toggling); whole FBP
+// of that stack 110 against 65 ms, 701^2 x 37 x 603 1.54 against 0.89.
+// The batch's form below keeps 45 registers in memory (all four widths of the
+// tile in one kernel of 128 registers), 64-slice tiles of 16 x 16 voxels three.
 #include "mr_bp.h"
 #include "mr_common.h"
 

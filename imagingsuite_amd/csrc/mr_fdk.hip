@@ -732,6 +732,11 @@ namespace mr {
 // more count as one: a padded group costs as much as a whole one, fdk_kernel
 // 1.3 times that for 256 slices at 1024^2) of volumes from 512^2: 256^2 x 256
 // x 360 takes 1.19 + 0.06 against 1.27 ms, 256^2 x 192 1.06 + 0.06 against 1.00.
+// Whole calls against fdk_kernel alone over 270 sizes: 0.83 to 1.01 for whole
+// groups from 600^2, mean 0.99 of all; padded ones and volumes just past 512,
+// whose partial patches count most, are on the other side of the line by up to a
+// fifth (224 slices: 513^2 1.14 to 1.20, 600^2 1.10, 1024^2 1.05 to 1.08; 513^2 x 256
+// to 300 1.02 to 1.12).
 static bool fdk_slice_shape(const mr_fdk_plan &p, const std::vector<float> &ptab, const std::vector<float> &zt1,
                             size_t w, size_t h, size_t np, FdkSliceArgs &a, size_t &lds)
 {

@@ -269,8 +269,10 @@ __global__ __launch_bounds__(256) void joseph_forward_lds_kernel(JosephArgs a, c
 // adds the column class's terms in another order: bit-identical to either.
 //
 // What limits it is the latency of a line (position, LDS address, LDS read,
-// barrier) at 3 to 5 waves per SIMD; the form before staged through registers
-// and read its spans when it needed them.  Projection in microseconds, before
+// barrier) at 3 to 5 waves per SIMD (512^2 x 16 x 360: LDS 43 % busy, 43 % of the
+// wave cycles waiting), and for volumes that do not stay in the caches their
+// fetch, once per chunk of angles (1024^2 x 64 x 900: 27 GB in 4.9 ms); the form
+// before staged through registers and read its spans when it needed them.  Projection in microseconds, before
 // and now: 512^2 x 16 x 360 (R = 2) 430, 260; 512^2 x 32 x 360 (R = 1) 567, 378
 // (502 with R = 2); 1024^2 x 64 x 200 5302, 3847 (4976 with R = 2); slice counts
 // that took joseph_forward_kernel: 300^2 x 20 x 200 461, 136; 700^2 x 8 x 200
@@ -467,14 +469,18 @@ __global__ __launch_bounds__(256) void joseph_adjoint_kernel(JosephArgs a)
 
 // LDS-staged adjoint: the structure of the parallel back-projector's tiled
 // kernel (16 x 16 voxel tile, ZT slices, C angles staged per chunk by direct
-// loads into one of two buffers while the other is summed, the XCD-striped tile
-// order) with the Joseph kernel K as weights.  For each angle the tile stages
+// loads into the other of two buffers, the XCD-striped tile order) with the Joseph
+// kernel K as weights.  For each angle the tile stages
 // the SPAN detector bins from floor(u) of its lowest corner, one bin of rounding
 // margin below; bins outside [0, n_det) are staged as zeros, which is where the
 // direct kernel's clamped loads have weight zero, and so are slices past the
-// last.  Bound by the LDS reads.  (Staged between two barriers per chunk:
-// 512^2 x 16 x 360 207 against 166 us, 512^2 x 32 x 360 358 against 272, 1024^2 x
-// 64 x 200 1.32 against 1.16 ms.)
+// last.  (Staged between two barriers per chunk: 512^2 x 16 x 360 207 against 166
+// us, 512^2 x 32 x 360 358 against 272, 1024^2 x 64 x 200 1.32 against 1.16 ms.)  As
+// there, the compiler waits for the loads ahead of a chunk's first read and the
+// CU's other blocks cover them (without that wait 0.94 to 1.03 times as long), and
+// no unit bounds it alone: 512^2 x 16 x 360 keeps the LDS busy for 53 % of the
+// cycles, issues 0.23 vector instructions per cycle and SIMD and waits for 36 %
+// of the wave cycles.
 constexpr int kJSpan = 26;
 
 template <int ZT, int C>
