@@ -272,11 +272,11 @@ __global__ __launch_bounds__(256) void joseph_forward_lds_kernel(JosephArgs a, c
 // barrier) at 3 to 5 waves per SIMD (512^2 x 16 x 360: LDS 43 % busy, 43 % of the
 // wave cycles waiting), and for volumes that do not stay in the caches their
 // fetch, once per chunk of angles (1024^2 x 64 x 900: 27 GB in 4.9 ms); the form
-// before staged through registers and read its spans when it needed them.  Projection in microseconds, before
-// and now: 512^2 x 16 x 360 (R = 2) 430, 260; 512^2 x 32 x 360 (R = 1) 567, 378
-// (502 with R = 2); 1024^2 x 64 x 200 5302, 3847 (4976 with R = 2); slice counts
-// that took joseph_forward_kernel: 300^2 x 20 x 200 461, 136; 700^2 x 8 x 200
-// (8 slices, R = 4) 924, 333.
+// before staged through registers and read its spans when it needed them.
+// Projection in microseconds, before and now: 512^2 x 16 x 360 (R = 2) 430, 260;
+// 512^2 x 32 x 360 (R = 1) 567, 378 (502 with R = 2); 1024^2 x 64 x 200 5302, 3847
+// (4976 with R = 2); slice counts that took joseph_forward_kernel: 300^2 x 20 x 200
+// 461, 136; 700^2 x 8 x 200 (8 slices, R = 4) 924, 333.
 // Dynamic LDS: N + 3 R spans.
 template <int ZT, int R>
 __global__ __launch_bounds__(256, R == 4 ? 4 : 5) void joseph_forward_dma_kernel(
@@ -470,9 +470,8 @@ __global__ __launch_bounds__(256) void joseph_adjoint_kernel(JosephArgs a)
 // LDS-staged adjoint: the structure of the parallel back-projector's tiled
 // kernel (16 x 16 voxel tile, ZT slices, C angles staged per chunk by direct
 // loads into the other of two buffers, the XCD-striped tile order) with the Joseph
-// kernel K as weights.  For each angle the tile stages
-// the SPAN detector bins from floor(u) of its lowest corner, one bin of rounding
-// margin below; bins outside [0, n_det) are staged as zeros, which is where the
+// kernel K as weights.  For each angle the tile stages the SPAN detector bins from
+// floor(u) of its lowest corner, one bin of rounding margin below; bins outside [0, n_det) are staged as zeros, which is where the
 // direct kernel's clamped loads have weight zero, and so are slices past the
 // last.  (Staged between two barriers per chunk: 512^2 x 16 x 360 207 against 166
 // us, 512^2 x 32 x 360 358 against 272, 1024^2 x 64 x 200 1.32 against 1.16 ms.)  As
