@@ -1313,7 +1313,7 @@ struct mr_bp_plan {
     int *d_idx = nullptr;
     float *d_w = nullptr;
     int impl = 1;  // 1 LDS-staged kernel, 0 direct-gather kernel
-    int stage64 = 0;  // 1: no matrix-core form (MR_BP_STAGE64 debug override)
+    bool no_matrix = false;  // no matrix-core form (MR_BP_STAGE64 debug override)
     size_t loaded_n = 0, loaded_nk = 0;   // projections / used projections of the resident tables
     bool loaded = false;
     void *d_adj = nullptr;                // adjoint chunks (int4) and projection order (int)
@@ -1337,8 +1337,8 @@ namespace mr {
 // whether a plan with nk used projections runs on the matrix cores
 static bool plan_bpm(const mr_bp_plan *p, size_t nk, int &tile)
 {
-    return p->p.fused && p->p.interp == MR_INTERP_LINEAR && p->impl == 1 && p->tilt == 0 && !p->stage64 && !p->no_split &&
-           bpm_shape((int)p->p.width, (int)p->p.slices, (int)nk, tile);
+    return p->p.fused && p->p.interp == MR_INTERP_LINEAR && p->impl == 1 && p->tilt == 0 && !p->no_matrix &&
+           !p->no_split && bpm_shape((int)p->p.width, (int)p->p.slices, (int)nk, tile);
 }
 }  // namespace mr
 
@@ -1441,7 +1441,7 @@ extern "C" int mr_bp_plan_create(mr_bp_plan **plan, const mr_bp_params *params)
     p->impl = (q.multiprojbp && (q.slices & 3)) ? 0 : 1;
     // debug override, read once per plan: MR_BP_STAGE64=1 keeps the fused form on
     // the vector kernel (whose staging takes 64-bit addresses at every size)
-    if (const char *e = std::getenv("MR_BP_STAGE64")) p->stage64 = std::atoi(e) == 1 ? 1 : 0;
+    if (const char *e = std::getenv("MR_BP_STAGE64")) p->no_matrix = std::atoi(e) == 1;
     mr::circle_mask(q.width, q.width, q.use_roi != 0, q.roi, false, p->first, p->second,
                     q.correct_tilt ? mr::tilt_mask_shrink(q.tilt_angle, q.tilt_rows) : 0.0f);
     std::vector<int2> m(q.width);
